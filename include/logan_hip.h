@@ -232,10 +232,10 @@ int logan_hip_affine_qmm(const LoganHipAffine *w, const void *x, int M, int x_st
 
 /* Up to 8 matrices that read the same x (q/k/v, qkvz/ba of a prefill
  * chunk) as one product: ys[i][M][O_i] = x . bf16(W_i)^T, each as
- * logan_hip_affine_qmm. With M >= 256 and power-of-two group sizes their
- * column tiles form one grid (the reference encodes its batch of products
- * into one command buffer, backend_metal.mm:2290-2493); otherwise one launch
- * per matrix. Every matrix has the same I, bits, group_size and aux type. 1
+ * logan_hip_affine_qmm. With 16-byte aligned weights (5-bit: 4-byte) and
+ * 4-byte aligned scales and biases their column tiles form one grid (the
+ * reference encodes its batch of products into one command buffer,
+ * backend_metal.mm:2290-2493); otherwise one launch per matrix. Every matrix has the same I, bits, group_size and aux type. 1
  * ok, 0 unsupported, -1 launch failure. Split grids share
  * logan_hip_affine_qmm's scratch slots and their cross-stream ordering. */
 int logan_hip_affine_qmm_multi(const LoganHipAffine *ws, int count, const void *x, int M,

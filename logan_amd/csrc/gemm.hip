@@ -4,17 +4,16 @@
 // dequantised weight rounded to bf16 in threadgroup memory, bf16 x bf16
 // products accumulated in f32, bf16 output).
 //
-// One block computes a 64 x 64 tile of y (4 waves, each a 32 x 32 tile with
-// v_mfma_f32_32x32x16_bf16). Per 64-wide k step the block dequantises its 64
-// weight rows into LDS (codes -> f32 fma -> v_cvt_pk_bf16_f32), while every
-// lane loads its x operands straight from global memory (x rows are re-read
-// by the N/64 blocks of a row block and stay in L2). Operand layout of the
-// 32x32x16 instruction (checked on the device): lane l holds row (col) l % 32
-// and 8 consecutive k at offset 8 * (l / 32) of each 16-wide k slice; the
-// result's element i of lane l is row 8 * (i / 4) + 4 * (l / 32) + i % 4,
-// column l % 32.
+// affine_qmm_tile_kernel serves every product whose rows allow 16-byte copies;
+// affine_qmm_kernel (64 x 64 tiles, 4 waves, dword loads) the rest (packed
+// rows off 16 bytes, scale / bias rows off 4) and the smallest products.
+// Operand layout of v_mfma_f32_32x32x16_bf16 (checked on the device): lane l
+// holds row (col) l % 32 and 8 consecutive k at offset 8 * (l / 32) of each
+// 16-wide k slice; the result's element i of lane l is row
+// 8 * (i / 4) + 4 * (l / 32) + i % 4, column l % 32.
 #include <algorithm>
 #include <atomic>
+#include <type_traits>
 
 #include "affine_dev.hpp"
 #include "lh_internal.hpp"
@@ -225,167 +224,44 @@ __global__ __launch_bounds__(256) void affine_qmm_kernel(GemmParams p, int kstep
   }
 }
 
-// ---------------------------------------------------------------------------
-// Large tiles: 128 x 128 output per 256-thread block (each wave 64 x 64 as
-// 2 x 2 MFMA tiles), so every weight is dequantised once per 128 tokens. Per
-// 64-k step the block writes the x tile and the dequantised W tile into one
-// of two LDS stages while the MFMAs read the other; the next step's global
-// loads are issued into registers before the current step's MFMAs, one
-// barrier per step. (x read straight into MFMA operand registers instead of
-// through LDS measured 1.7x slower: each load instruction then touches 32
-// rows.) Blocks are numbered so that the M tiles of one N tile share an XCD
-// (block id mod 8) and meet the weight tile in that XCD's L2.
-constexpr int kQ2 = 128;     // tile rows (m) and columns (n)
-constexpr int kQ2Ld = 72;    // bf16 per LDS row: 64 + 8 pad
-#ifndef QMM_MIN_TILES
-#define QMM_MIN_TILES 192
-#endif
-constexpr int kQ2MinTiles = QMM_MIN_TILES;
 constexpr int kQTargetBlocks = 512;  // about two blocks per CU
 static SlotRing g_qmm_slots(kQSlots);
 
-template <int BITS>
-__global__ __launch_bounds__(256) void affine_qmm128_kernel(GemmParams p, int mtiles, int ntiles,
-                                                            int ksteps, int slot) {
-  // two stages: step s reads stage s % 2 while stage (s + 1) % 2 is filled
-  __shared__ __align__(16) __bf16 sA[2][kQ2 * kQ2Ld];
-  __shared__ __align__(16) __bf16 sB[2][kQ2 * kQ2Ld];
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave >> 1, wn = wave & 1;
-  const int half = lane >> 5, l32 = lane & 31;
-  // XCD-grouped tile order
-  const int L = blockIdx.x;
-  const int grp = L / (8 * mtiles), rem = L % (8 * mtiles);
-  const int nt = grp * 8 + rem % 8, mt = rem / 8;
-  if (nt >= ntiles) return;
-  const int bm0 = mt * kQ2, bn0 = nt * kQ2;
-
-  // loader role: row lr of both tiles, codes / activations [32 lh, 32 lh + 32)
-  const int lr = tid >> 1, lh = tid & 1;
-  const uint16_t *xrow = p.x + (size_t)min(bm0 + lr, p.M - 1) * p.x_stride + 32 * lh;
-  const int wrw = min(bn0 + lr, p.N - 1);
-  const uint8_t *wrow = p.w + (size_t)wrw * p.row_bytes;
-  const uint16_t *srow = p.sc + (size_t)wrw * p.ng;
-  const uint16_t *brow = p.bi + (size_t)wrw * p.ng;
-  struct Loads {
-    uint4 x0, x1, x2, x3;
-    uint32_t w[BITS];
-    uint32_t s, b;
-  };
-  auto issue = [&](int k0) {
-    Loads r;
-    const uint4 *xs = reinterpret_cast<const uint4 *>(xrow + k0);
-    r.x0 = xs[0];
-    r.x1 = xs[1];
-    r.x2 = xs[2];
-    r.x3 = xs[3];
-    load_chunk<BITS>(r.w, wrow + (size_t)(k0 + 32 * lh) * BITS / 8);
-    const int gi = (k0 + 32 * lh) / p.gs;
-    r.s = srow[gi];
-    r.b = brow[gi];
-    return r;
-  };
-  auto commit = [&](const Loads &r, int st) {
-    uint4 *da = reinterpret_cast<uint4 *>(sA[st] + lr * kQ2Ld + 32 * lh);
-    da[0] = r.x0;
-    da[1] = r.x1;
-    da[2] = r.x2;
-    da[3] = r.x3;
-    const float s = aux_to_f32_sel(r.s, p.fp16), b = aux_to_f32_sel(r.b, p.fp16);
-    uint32_t pk[16];
-#pragma unroll
-    for (int j = 0; j < 32; j += 2) {
-      // codes j, j + 1 of the 32-code chunk (LSB-first stream)
-      uint32_t c[2];
-#pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        const int bit = (j + q) * BITS, i = bit >> 5, sh = bit & 31;
-        uint32_t v = r.w[i] >> sh;
-        if (sh + BITS > 32) v |= r.w[i + 1] << (32 - sh);
-        c[q] = v & ((1u << BITS) - 1u);
-      }
-      bf16x2 v;
-      v[0] = (__bf16)fmaf((float)c[0], s, b);
-      v[1] = (__bf16)fmaf((float)c[1], s, b);
-      pk[j / 2] = __builtin_bit_cast(uint32_t, v);
-    }
-    uint4 *db = reinterpret_cast<uint4 *>(sB[st] + lr * kQ2Ld + 32 * lh);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) db[v] = make_uint4(pk[4 * v], pk[4 * v + 1], pk[4 * v + 2], pk[4 * v + 3]);
-  };
-
-  f32x16 acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = f32x16{};
-  auto mfma_step = [&](int st) {
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      bf16x8 a[2], b[2];
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-        a[i] = *reinterpret_cast<const bf16x8 *>(sA[st] + (wm * 64 + 32 * i + l32) * kQ2Ld + 16 * ks +
-                                                 8 * half);
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-        b[j] = *reinterpret_cast<const bf16x8 *>(sB[st] + (wn * 64 + 32 * j + l32) * kQ2Ld + 16 * ks +
-                                                 8 * half);
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
-    }
-  };
-  // per step: the MFMAs read stage s % 2 while the next step's operands
-  // (loaded during the previous step) are dequantised into the other stage,
-  // then the loads of step s + 2 are issued; one barrier per step (stage
-  // (s + 1) % 2 was last read in step s - 1, before that step's barrier).
-  // (Loads issued three steps ahead measured no faster.)
-  const int z = blockIdx.y;
-  const int kb = z * ksteps * 64, nst = (min(p.K, kb + ksteps * 64) - kb) / 64;
-  Loads cur = issue(kb);
-  commit(cur, 0);
-  cur = issue(kb + 64 * min(1, nst - 1));
-  __syncthreads();
-  for (int s = 0; s < nst; ++s) {
-    mfma_step(s & 1);
-    if (s + 1 < nst) {
-      commit(cur, (s + 1) & 1);
-      cur = issue(kb + 64 * min(s + 2, nst - 1));
-    }
-    __syncthreads();
-  }
-  // element e of tile (i, j): row 32 i + 8 (e / 4) + 4 half + e % 4, column 32 j + l32
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int n = bn0 + wn * 64 + 32 * j + l32;
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const int m = bm0 + wm * 64 + 32 * i + 8 * (e / 4) + 4 * half + (e % 4);
-        if (m < p.M && n < p.N) qmm_store(p, slot, z, m, n, acc[i][j][e]);
-      }
-    }
-}
-
 // ---------------------------------------------------------------------------
-// 256 x 128 tiles for M >= 256, over up to kQMultiMax matrices that read the
-// same x (q/k/v, qkvz/ba) in one grid. 512 threads, waves 4 (m) x 2 (n), each
-// 64 x 64 as 2 x 2 v_mfma_f32_32x32x16_bf16 tiles, so every dequantised weight
-// serves 256 tokens (half the VALU per MFMA of the 128-row tiles).
-//   * step s's x rows and the codes / scale / bias of its weights are loaded
-//     into one of two register sets two steps ahead, then written to LDS
-//     stage s & 1 (the weights dequantised to bf16) one step ahead, and
-//     multiplied after the barrier that follows: one barrier per step, and
-//     the loads of the next two steps stay in flight across it;
-//   * LDS rows are 144 bytes (64 bf16 + 16 bytes of padding), so the 16
-//     lanes an operand read serves per clock (rows r .. r + 15 at one k
-//     offset) start on 16 different 4-bank groups of the 64 banks.
-constexpr int kQ3M = 256, kQ3N = 128;
-constexpr int kQ3Ld = 72;  // u16 per LDS row: 64 + 8 of padding
+// Products of up to kQMultiMax matrices that read the same x (q/k/v, qkvz/ba,
+// gate/up) in one grid, BM x 128 output tiles, one 8-wave block per CU.
+//
+// What bounds it: 256-row tiles the vector and matrix pipes together (per
+// 64-k step and SIMD 1024 cycles of MFMA and about 600 issue cycles of VALU,
+// most of it the forming of the bf16 weights); tiles of at most 128 rows the
+// forming alone and, at 8 bits, the stream of codes from HBM. Hence:
+//   * every copy from memory goes straight into LDS (global_load_lds, issued
+//     through inline assembly and waited for by count) NST - 1 steps ahead: x
+//     rows, packed codes, and the scale / bias words a chunk of steps at a
+//     time. No VGPR holds a load in flight, and every line is read whole;
+//   * the weights never go back to LDS: a lane reads its run of codes, forms
+//     bf16(code * scale + bias) in the MFMA operand's layout and feeds it to
+//     all MI = BM / 32 row tiles. The 8 waves are 4 (32 columns each) x 2 (k
+//     halves of each step), so every weight is formed once per block; the two
+//     waves of a tile add their sums through LDS after the last step;
+//   * the copies of a step are issued between its MFMAs, at the places the
+//     scheduling barriers fix: issued together at its start they hold the
+//     waves at the CU's one address path before their first MFMA (2 x 14336
+//     columns, 8-bit, K 4096, M 2048: 600 us so, 551 us spread).
+// Measured, us (before: 256 x 128 tiles with the weights staged in LDS as bf16,
+// 128 x 128 below 256 rows, one launch per matrix there):
+//   8-bit, 2 x 14336 x 4096: M 100  88.0 -> 47.2, M 2048  619 -> 520 (925 TFLOP/s)
+//   8-bit, 4096 x 14336:     M 100  44.6 -> 34.3, M 2048  284 -> 235
+//   4-bit, 12352 x 2048:     M 512  41.3 -> 36.2;  9216 x 2048: 39.0 -> 30.5
+//   4-bit, 2048 x 4096:      M 512  26.7 -> 25.4 (with the reduction)
+// Within a step, wave k-group kg and lane half h own the run of 16 codes at
+// k = 16 (2 kg + h), and MFMA slice j takes 8 of them: any order of k serves
+// as long as both operands use it.
+// LDS: x rows are 128 bytes, 16-byte granule q of row r at q ^ ((r >> 1) & 7)
+// (16 rows of an operand read spread over all banks: no conflicts counted);
+// 8-bit codes likewise at q ^ ((r >> 2) & 3) of their 64 bytes; the narrower
+// rows need no swizzle.
+constexpr int kTN = 128;   // tile columns
 constexpr int kQMultiMax = 8;
 
 struct QmmMat {
@@ -394,115 +270,510 @@ struct QmmMat {
   const uint16_t *bi;
   void *y;
   long long row_bytes;
-  int N, ng, y_stride, col0;  // col0: first column of this matrix in split partial rows
+  int N, ng, y_stride, col0;  // col0: first column of this matrix in split partial rows (a multiple of 4)
 };
 struct QmmMulti {
   QmmMat m[kQMultiMax];
   int tile_start[kQMultiMax + 1];  // first 128-column tile of matrix i
   const uint16_t *x;
   int n, M, K, gs, fp16, x_stride, y_bf16, part_N;
-  int vec;  // bit 0: y rows take 16-byte stores; bit 1: partial rows do
+  int vec;  // y rows take 16-byte stores
 };
 
-template <int BITS>
-struct Q3Raw {
-  uint32_t w[BITS == 4 ? 2 : BITS == 8 ? 4 : 3];
-  uint32_t s, b;
-};
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t q3_rsrc(const void *p, long long bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), (short)0,
-                                           (int)(bytes > 0x7fffffffLL ? 0x7fffffffLL : bytes),
-                                           0x00020000);
+__device__ __forceinline__ uint32_t q_lds_addr(const void *p) {
+  return (uint32_t)(uintptr_t)((__attribute__((address_space(3))) const uint8_t *)p);
 }
-
-// 16 codes [k, k + 16) of a row (k a multiple of 16) and their group's scale
-// and bias: exactly three buffer loads
-template <int BITS>
-__device__ __forceinline__ void q3_load(Q3Raw<BITS> &r, __amdgpu_buffer_rsrc_t wr,
-                                        __amdgpu_buffer_rsrc_t sr, __amdgpu_buffer_rsrc_t br,
-                                        int rowoff, int poff, int k) {
-  if constexpr (BITS == 4) {
-    const uint2 v = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(wr, rowoff + (k >> 1), 0, 0));
-    r.w[0] = v.x;
-    r.w[1] = v.y;
-  } else if constexpr (BITS == 8) {
-    const uint4 v = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(wr, rowoff + k, 0, 0));
-    r.w[0] = v.x;
-    r.w[1] = v.y;
-    r.w[2] = v.z;
-    r.w[3] = v.w;
-  } else {
-    typedef uint32_t u32x3 __attribute__((ext_vector_type(3)));
-    const u32x3 v = __builtin_bit_cast(
-        u32x3, __builtin_amdgcn_raw_buffer_load_b96(wr, rowoff + 4 * ((k * BITS) >> 5), 0, 0));
-    r.w[0] = v.x;
-    r.w[1] = v.y;
-    r.w[2] = v.z;
-  }
-  r.s = __builtin_amdgcn_raw_buffer_load_b16(sr, poff, 0, 0);
-  r.b = __builtin_amdgcn_raw_buffer_load_b16(br, poff, 0, 0);
+// lane l's 16 (4, 2) bytes at base + off land at lds + 16 l (4 l; the 2 as a
+// zero-extended dword); lds and base are wave-uniform. Completion counts in vmcnt, unseen by the compiler.
+__device__ __forceinline__ void q_copy16(const void *base, uint32_t off, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+               :: "v"(off), "s"(base), "s"(lds) : "memory", "m0");
 }
-
-// bf16(code * s + b) of the 16 codes, packed in pairs (code order); sh is the
-// bit where the first 5-bit code starts (0 or 16)
-template <int BITS>
-__device__ __forceinline__ void q3_dequant(const Q3Raw<BITS> &r, int sh, bool fp16, uint32_t (&pk)[8]) {
-  const float s = aux_to_f32_sel(r.s, fp16), b = aux_to_f32_sel(r.b, fp16);
-  float f[16];
-  if constexpr (BITS == 4) {
-#pragma unroll
-    for (int d = 0; d < 2; ++d) {
-      const uint32_t lo = r.w[d] & 0x0F0F0F0Fu, hi = (r.w[d] >> 4) & 0x0F0F0F0Fu;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        f[8 * d + 2 * i] = (float)((lo >> (8 * i)) & 255u);
-        f[8 * d + 2 * i + 1] = (float)((hi >> (8 * i)) & 255u);
-      }
-    }
-  } else if constexpr (BITS == 8) {
-#pragma unroll
-    for (int d = 0; d < 4; ++d)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) f[4 * d + i] = (float)((r.w[d] >> (8 * i)) & 255u);
-  } else {
-    const uint32_t win[3] = {__builtin_amdgcn_alignbit(r.w[1], r.w[0], sh),
-                             __builtin_amdgcn_alignbit(r.w[2], r.w[1], sh), r.w[2] >> sh};
-#pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      const int bit = j * BITS, i = bit >> 5, o = bit & 31;
-      uint32_t v = win[i] >> o;
-      if (o + BITS > 32) v |= win[i + 1] << (32 - o);
-      f[j] = (float)(v & ((1u << BITS) - 1u));
-    }
-  }
-#pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    bf16x2 v;
-    v[0] = (__bf16)fmaf(f[2 * j], s, b);
-    v[1] = (__bf16)fmaf(f[2 * j + 1], s, b);
-    pk[j] = __builtin_bit_cast(uint32_t, v);
-  }
+__device__ __forceinline__ void q_copy4(const void *base, uint32_t off, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1"
+               :: "v"(off), "s"(base), "s"(lds) : "memory", "m0");
 }
-
+__device__ __forceinline__ void q_copy2(const void *base, uint32_t off, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_ushort %0, %1"
+               :: "v"(off), "s"(base), "s"(lds) : "memory", "m0");
+}
 template <int N>
-__device__ __forceinline__ void q3_wait() {
+__device__ __forceinline__ void q_wait() {
+  static_assert(N >= 0 && N <= 63, "vmcnt is 6 bits");
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
+// Geometry of one instantiation.
+template <int BITS, int MI, bool GS64>
+struct QTile {
+  static constexpr int BM = 32 * MI;               // tile rows
+  static constexpr int RB = 8 * BITS;              // code bytes per row and step
+  static constexpr int XB = BM * 128;              // x bytes per stage
+  static constexpr int WB = kTN * RB;
+  // stages of x and of the codes (a step's codes are read a step ahead of its x)
+  static constexpr int NST = BM >= 192 ? 4 : BM == 128 ? 5 : 8;
+  static constexpr int NWS = NST - 1;
+  static constexpr int AUX0 = NST * XB + NWS * WB;
+  // steps of a chunk of scale / bias words, dwords per row of it: CS groups of
+  // 64 that may start inside a dword; groups of 32 start on one
+  static constexpr int ndw(int cs) { return GS64 ? cs / 2 + 1 : cs; }
+  static constexpr int ab(int cs) { return 2 * kTN * ndw(cs) * 4; }  // [scale, bias][128][ndw]
+  static constexpr int CS = AUX0 + 2 * ab(8) <= 163840 ? 8 : AUX0 + 2 * ab(6) <= 163840 ? 6 : 4;
+  static constexpr int NDW = ndw(CS);
+  static constexpr int AB = ab(CS);
+  static constexpr int XI = BM / 8;                // x copies (1 KB) of a stage
+  static constexpr int LX = (XI + 7) / 8;          // per wave
+  static constexpr int WI = BITS == 5 ? 20 : BITS; // code copies (1 KB; 5-bit 256 bytes)
+  static constexpr int LW = (WI + 7) / 8;
+  static constexpr int L = LX + LW;
+  static constexpr int NA = (4 * NDW + 7) / 8;     // scale / bias copies per wave and chunk
+  static constexpr int RINGS = AUX0 + 2 * AB;
+  // sum exchange: a 32 x 32 tile per wave; stores: one of 33-float rows
+  static constexpr int ROUND = 8 * 4096 + 8 * 32 * 33 * 4;
+  static constexpr int BYTES = RINGS > ROUND ? RINGS : ROUND;
+  static_assert(BYTES <= 163840 && CS >= NST, "ring geometry");
+  static_assert((NST - 2) * L + NA <= 63, "vmcnt is 6 bits");
+};
+
+// wait until all but the last n * L (n <= MAX, uniform) copies of this wave have landed
+template <int L, int MAX>
+__device__ __forceinline__ void q_wait_steps(int n) {
+  if constexpr (MAX > 0) {
+    if (n >= MAX) q_wait<MAX * L>();
+    else q_wait_steps<L, MAX - 1>(n);
+  } else {
+    q_wait<0>();
+  }
+}
+
+// the lane's run of 16 codes from its row's RB bytes in LDS
+template <int BITS>
+struct QRun {
+  uint32_t w[BITS == 4 ? 2 : BITS == 8 ? 4 : 3];
+  __device__ __forceinline__ void read(const uint8_t *row, int r, int run) {
+    if constexpr (BITS == 8) {
+      const uint4 v = *reinterpret_cast<const uint4 *>(row + ((run ^ ((r >> 2) & 3)) << 4));
+      w[0] = v.x;
+      w[1] = v.y;
+      w[2] = v.z;
+      w[3] = v.w;
+    } else if constexpr (BITS == 4) {
+      const uint2 v = *reinterpret_cast<const uint2 *>(row + 8 * run);
+      w[0] = v.x;
+      w[1] = v.y;
+    } else {
+      // the dword holding the first code on; 5-bit codes may start at its bit 16
+      const uint32_t *p = reinterpret_cast<const uint32_t *>(row + ((2 * BITS * run) & ~3));
+#pragma unroll
+      for (int i = 0; i < 3; ++i) w[i] = p[i];
+    }
+  }
+  // codes 8 j + 2 i, + 1 as f32 (from what split() left)
+  __device__ __forceinline__ void split(int j, int sh, uint32_t (&t)[3]) const {
+    if constexpr (BITS == 4) {
+      // (asm: the compiler would undo the two masks into a shift and a mask per code)
+      t[1] = w[j] >> 4;
+      asm("v_and_b32 %0, 0xf0f0f0f, %1" : "=v"(t[0]) : "v"(w[j]));
+      asm("v_and_b32 %0, 0xf0f0f0f, %0" : "+v"(t[1]));
+    } else if constexpr (BITS == 8) {
+      t[0] = w[2 * j];
+      t[1] = w[2 * j + 1];
+    } else if constexpr (BITS == 5) {
+      // sh: bit of the run's first code in w[0] (0 or 16)
+      t[0] = __builtin_amdgcn_alignbit(w[1], w[0], sh);
+      t[1] = __builtin_amdgcn_alignbit(w[2], w[1], sh);
+      t[2] = w[2] >> sh;
+    } else {
+#pragma unroll
+      for (int i = 0; i < 3; ++i) t[i] = w[i];
+    }
+  }
+  // bf16(code * s + b) of codes 8 j + 2 i, + 1, packed
+  static __device__ __forceinline__ uint32_t pair(const uint32_t (&t)[3], int j, int i, float s, float b) {
+    float f[2];
+    if constexpr (BITS == 4) {
+      f[0] = (float)((t[0] >> (8 * i)) & 255u);
+      f[1] = (float)((t[1] >> (8 * i)) & 255u);
+    } else if constexpr (BITS == 8) {
+      f[0] = (float)((t[i >> 1] >> (16 * (i & 1))) & 255u);
+      f[1] = (float)((t[i >> 1] >> (16 * (i & 1) + 8)) & 255u);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const int bit = (8 * j + 2 * i + e) * BITS, q = bit >> 5, o = bit & 31;
+        uint32_t v = t[q] >> o;
+        if (o + BITS > 32) v |= t[q + 1] << (32 - o);
+        f[e] = (float)(v & ((1u << BITS) - 1u));
+      }
+    }
+    bf16x2 v;
+    v[0] = (__bf16)fmaf(f[0], s, b);
+    v[1] = (__bf16)fmaf(f[1], s, b);
+    return __builtin_bit_cast(uint32_t, v);
+  }
+};
+
+// GS64: groups of 64 codes (a group per step); else any multiple of 32
+template <int BITS, int MI, bool GS64, bool FP16>
+__global__ __launch_bounds__(512, 2) void affine_qmm_tile_kernel(QmmMulti p, int mtiles, int ntiles,
+                                                                 int ksteps, int slot) {
+  using G = QTile<BITS, MI, GS64>;
+  constexpr int BM = G::BM, NST = G::NST, CS = G::CS, NDW = G::NDW;
+  __shared__ __align__(256) uint8_t smem[G::BYTES];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wn = wave & 3, kg = wave >> 2;
+  const int half = lane >> 5, l32 = lane & 31;
+  // Block order: each XCD (block id mod 8) takes one run of the tiles, row tiles
+  // fastest, so that the row tiles of one (column tile, k range) meet its
+  // weights in one L2 and every XCD has as many blocks to within one
+  const int total = mtiles * ntiles * ((p.K / 64 + ksteps - 1) / ksteps);
+  const int lin = (int)(blockIdx.x & 7) * ((total + 7) / 8) + (int)(blockIdx.x >> 3);
+  if (lin >= total) return;
+  const int mt = lin % mtiles, col = lin / mtiles;
+  const int nt = col % ntiles, z = col / ntiles;
+  int mi = 0;
+#pragma unroll
+  for (int t = 1; t < kQMultiMax; ++t) mi = t < p.n && nt >= p.tile_start[t] ? t : mi;
+  mi = __builtin_amdgcn_readfirstlane(mi);
+  const QmmMat &mat = p.m[mi];
+  const int bm0 = mt * BM, bn0 = (nt - p.tile_start[mi]) * kTN;
+  const int kb = z * ksteps * 64;
+  int nst = (min(p.K, kb + ksteps * 64) - kb) >> 6;
+  // the arguments the loop uses, kept in registers (the copies' memory
+  // clobbers would have them loaded again, and waited for, in every step)
+  int N = mat.N, ng = mat.ng, gs = p.gs;
+  const uint16_t *sc = mat.sc, *bi = mat.bi;
+  asm volatile("" : "+s"(N), "+s"(ng), "+s"(gs), "+s"(sc), "+s"(bi), "+s"(nst));
+
+  // ---- this wave's copies: of every stage, LX of x and LW of the codes ----
+  uint32_t xoff[G::LX], woff[G::LW], wdst[G::LW];
+  const uint32_t lds0 = __builtin_amdgcn_readfirstlane(q_lds_addr(smem));
+  const uint32_t xdst = lds0 + 1024 * ((wave * G::LX) % G::XI);
+#pragma unroll
+  for (int i = 0; i < G::LX; ++i) {
+    const int r = 8 * ((wave * G::LX + i) % G::XI) + (lane >> 3);  // copies past the tile repeat one
+    const int g = (lane & 7) ^ ((r >> 1) & 7);
+    xoff[i] = (uint32_t)(min(r, p.M - 1 - bm0) * p.x_stride + 8 * g) * 2u;
+  }
+#pragma unroll
+  for (int i = 0; i < G::LW; ++i) {
+    const int c = (wave * G::LW + i) % G::WI, u = 64 * c + lane;
+    int r, b;
+    if constexpr (BITS == 5) {
+      r = u / 10;
+      b = 4 * (u % 10);
+    } else {
+      r = u / (G::RB / 16);
+      const int q = u % (G::RB / 16);
+      b = 16 * (BITS == 8 ? q ^ ((r >> 2) & 3) : q);
+    }
+    woff[i] = (uint32_t)(min(r, N - 1 - bn0) * (int)mat.row_bytes + b);
+    wdst[i] = lds0 + NST * G::XB + (BITS == 5 ? 256 : 1024) * c;
+  }
+  const uint8_t *xsrc = reinterpret_cast<const uint8_t *>(p.x + (size_t)bm0 * p.x_stride + kb);
+  const uint8_t *wsrc = mat.w + (size_t)bn0 * mat.row_bytes + (size_t)kb * BITS / 8;
+  // the next step's copy k of L, into the stages at bytes xst, wst of the rings
+  int xst = 0, wst = 0;
+  auto copy = [&](int k) __attribute__((always_inline)) {
+    if (k < G::LX) {
+      const int i = k < G::LX ? k : 0;
+      q_copy16(xsrc, xoff[i], xdst + xst + 1024 * i);
+    } else {
+      const int i = k < G::LX ? 0 : k - G::LX;
+      if constexpr (BITS == 5) q_copy4(wsrc, woff[i], wdst[i] + wst);
+      else q_copy16(wsrc, woff[i], wdst[i] + wst);
+    }
+  };
+  auto next = [&]() __attribute__((always_inline)) {
+    xsrc += 128;
+    wsrc += G::RB;
+    xst = xst == (NST - 1) * G::XB ? 0 : xst + G::XB;
+    wst = wst == (G::NWS - 1) * G::WB ? 0 : wst + G::WB;
+  };
+  // Scale / bias words: chunks of CS steps, the ndw dwords of each row that
+  // hold the chunk's groups (from the dword with the first one on: rows of an
+  // odd number of groups start inside a dword), in two buffers. 64
+  // consecutive dwords of a chunk's [scale, bias][128][ndw] are one copy.
+  const bool g32 = !GS64 && gs == 32;
+  const int ndw = GS64 || g32 ? NDW : CS / 2 + 1;
+  const uint32_t ldsa = lds0 + G::AUX0;
+  // the last dword wholly inside the matrix; when the total is odd, the word
+  // after it is copied alone (zero-extended)
+  const uint32_t atot = (uint32_t)N * ng * 2u, amax = (atot & ~3u) - 4u;
+  const bool odd = (atot & 2u) != 0 && bn0 + kTN >= N;
+  auto aux_chunk = [&](int c) __attribute__((always_inline)) {
+    const int k = kb + 64 * CS * c;
+    const uint32_t g0 = GS64 ? (uint32_t)k >> 6 : (uint32_t)k / (uint32_t)gs;
+    const int per = 2 * ndw;  // copies of the scales (128 ndw / 64), then the biases'
+#pragma unroll
+    for (int i = 0; i < G::NA; ++i) {
+      int s = wave * G::NA + i;  // copies past the chunk repeat one
+      s = s >= 2 * per ? s - 2 * per : s;
+      const bool bias = s >= per;
+      const uint32_t d = 64 * (bias ? s - per : s) + lane;
+      const uint32_t r = GS64 ? d / NDW : g32 ? d / NDW : d / (CS / 2 + 1);
+      const uint32_t u16i = ((uint32_t)min(bn0 + (int)r, N - 1) * ng + g0) & ~1u;
+      const uint32_t o = 2 * u16i + 4 * (d - r * ndw);
+      const uint16_t *src = bias ? bi : sc;
+      const uint32_t dst = __builtin_amdgcn_readfirstlane(ldsa + (c & 1) * G::AB + 256 * s);
+      if (!odd) {
+        q_copy4(src, min(o, amax), dst);
+      } else {
+        // (waited for at once: its copies would not be the NA counted)
+        if (o == atot - 2) q_copy2(src, o, dst);
+        else q_copy4(src, min(o, amax), dst);
+        q_wait<0>();
+      }
+    }
+  };
+
+  // ---- operands ----
+  const int run = 2 * kg + half;
+  const int nrow = wn * 32 + l32;
+  const uint8_t *xrd[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) xrd[j] = smem + l32 * 128 + (((2 * run + j) ^ ((l32 >> 1) & 7)) << 4);
+  const uint8_t *wrd = smem + NST * G::XB + nrow * G::RB;
+  const uint8_t *ard = smem + G::AUX0 + nrow * (4 * ndw);
+  const int par = ((bn0 + nrow) * ng) & 1;
+  const int sh = BITS == 5 ? 16 * (run & 1) : 0;
+
+  f32x16 acc[MI];
+#pragma unroll
+  for (int i = 0; i < MI; ++i) acc[i] = f32x16{};
+
+  struct Raw {
+    QRun<BITS> c;
+    uint32_t s, b;
+    __device__ __forceinline__ float scale() const { return FP16 ? f16_to_f32(s) : bf16_to_f32(s); }
+    __device__ __forceinline__ float bias() const { return FP16 ? f16_to_f32(b) : bf16_to_f32(b); }
+  };
+  // The next step's scale / bias words: GS64: two bytes on per step, and at a
+  // chunk's first step to the other buffer and the word its first group
+  // starts at. Other sizes (32-code groups: two per step; the rest at most
+  // one): where the group of the runs' half of the step is, counted from the
+  // chunk's first.
+  const int gse = GS64 || g32 ? 64 : gs, ginc = g32 ? 2 : 1;
+  const int ablk = GS64 ? 0 : 32 * kg;
+  int rt = 0;  // the next step
+  int cgr = GS64 ? kb >> 6 : kb / gs;         // first group of the next step
+  int rgr = GS64 ? cgr : (kb + ablk) / gs;    // and of its runs
+  int crem = GS64 || g32 ? 0 : kb % gs, rrem = GS64 || g32 ? 0 : (kb + ablk) % gs;
+  int cg0 = cgr;
+  auto read_raw = [&](int wo, Raw &r) __attribute__((always_inline)) {
+    const int c = rt / CS;
+    if (rt == c * CS) cg0 = cgr;
+    const uint8_t *ap = ard + ((c & 1) * G::AB + 2 * (rgr - cg0)) + 2 * ((par + cg0) & 1);
+    r.c.read(wrd + wo, l32, run);
+    r.s = *reinterpret_cast<const uint16_t *>(ap);
+    r.b = *reinterpret_cast<const uint16_t *>(ap + kTN * 4 * ndw);
+    ++rt;
+    if constexpr (GS64) {
+      ++cgr;
+      ++rgr;
+    } else {
+      crem += 64;
+      rrem += 64;
+      const bool n0 = crem >= gse, n1 = rrem >= gse;
+      cgr += n0 ? ginc : 0;
+      rgr += n1 ? ginc : 0;
+      crem -= n0 ? gse : 0;
+      rrem -= n1 ? gse : 0;
+    }
+  };
+  // Pipeline. Step t's iteration waits for its own copies of step t + 1 (those
+  // of the NST - 3 steps after it may be in flight), meets the barrier (step
+  // t + 1 is then readable, and nobody reads x of step t - 1 or codes of step t
+  // any more) and, between its MFMAs, issues the copies of step t + NST - 1; a
+  // chunk's first step also copies the next chunk's scale / bias words. While
+  // the MFMAs of one k slice run, the next slice's weights are formed and each
+  // x operand is read again, for the next slice, as soon as its MFMA has taken
+  // it: across the step's end too. The order is fixed by scheduling barriers:
+  // copies issued together at the step's start hold the waves at the CU's
+  // one address path (40 KB take about 640 cycles) before their first MFMA.
+  aux_chunk(0);
+  for (int t = 0; t < NST - 1 && t < nst; ++t) {
+#pragma unroll
+    for (int k = 0; k < G::L; ++k) copy(k);
+    next();
+  }
+  q_wait_steps<G::L, NST - 2>(min(NST - 2, nst - 1));
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_sched_barrier(0);
+  Raw raw;
+  bf16x8 xa[MI];
+  uint32_t wf[2][4];
+  read_raw(0, raw);
+#pragma unroll
+  for (int i = 0; i < MI; ++i) xa[i] = *reinterpret_cast<const bf16x8 *>(xrd[0] + 4096 * i);
+  {
+    uint32_t tw[3];
+    raw.c.split(0, sh, tw);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) wf[0][i] = QRun<BITS>::pair(tw, 0, i, raw.scale(), raw.bias());
+  }
+  int so = 0, wo = 0, cs = 0;  // stages of step t; t % CS
+  auto step = [&](auto copies, int t) __attribute__((always_inline)) {
+    constexpr bool COPY = decltype(copies)::value;
+    cs = cs == CS - 1 ? 0 : cs + 1;
+    const int sn = so == (NST - 1) * G::XB ? 0 : so + G::XB;
+    wo = wo == (G::NWS - 1) * G::WB ? 0 : wo + G::WB;
+    __builtin_amdgcn_sched_barrier(0);
+    // (past the last step: a stage of older data, read and not used)
+    Raw nraw;
+    read_raw(wo, nraw);
+    int k = 0;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      if (COPY && j == 1 && cs == 1) aux_chunk(t / CS + 1);
+      const Raw &r = j == 0 ? raw : nraw;
+      const uint8_t *xp = j == 0 ? xrd[1] + so : xrd[0] + sn;
+      const bf16x8 wv = __builtin_bit_cast(bf16x8, make_uint4(wf[j][0], wf[j][1], wf[j][2], wf[j][3]));
+      uint32_t tw[3];
+#pragma unroll
+      for (int i = 0; i < MI; ++i) {
+        acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wv, xa[i], acc[i], 0, 0, 0);
+        xa[i] = *reinterpret_cast<const bf16x8 *>(xp + 4096 * i);
+        // the last slice's codes come from LDS at the step's start: not first thing
+        constexpr int P0 = MI > 4 ? MI - 4 : 0;
+        if (i == P0) r.c.split(j ^ 1, sh, tw);
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          if (i == min(P0 + q, MI - 1)) wf[j ^ 1][q] = QRun<BITS>::pair(tw, j ^ 1, q, r.scale(), r.bias());
+        if constexpr (COPY) {
+#pragma unroll
+          for (int c = 0; c < G::L; ++c)
+            if (c >= k && c < ((j * MI + i + 1) * G::L) / (2 * MI)) copy(c);
+          k = ((j * MI + i + 1) * G::L) / (2 * MI);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    if constexpr (COPY) next();
+    raw = nraw;
+    so = sn;
+  };
+  int t = 0;
+  for (; t + NST - 1 < nst; ++t) {
+    __builtin_amdgcn_sched_barrier(0);
+    if ((unsigned)(cs - 1) < (unsigned)(NST - 3)) q_wait<(NST - 3) * G::L + G::NA>();
+    else q_wait<(NST - 3) * G::L>();
+    __builtin_amdgcn_s_barrier();
+    step(std::true_type{}, t);
+  }
+  for (; t < nst; ++t) {
+    __builtin_amdgcn_sched_barrier(0);
+    q_wait<0>();
+    __builtin_amdgcn_s_barrier();
+    step(std::false_type{}, t);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+
+  // ---- sums of the two waves of a tile, added in k order, and stores ----
+  // Element e of a 32 x 32 tile in lane l: column (m) l % 32, row (n)
+  // 8 (e / 4) + 4 (l / 32) + e % 4, so a lane stores 4 consecutive columns of
+  // y at a time. Row tile i is summed and stored by k-group i % 2.
+  const bool split = slot >= 0;
+  float *part = split ? g_qmm_part + (size_t)slot * kQSlotFloats + (size_t)z * p.M * p.part_N + mat.col0
+                      : nullptr;
+  float *const flat = reinterpret_cast<float *>(smem + 32768 + wave * (32 * 33 * 4));
+  auto store = [&](int i, const f32x16 &v) {
+    const int m = bm0 + 32 * i + l32, nw = bn0 + wn * 32;
+    if (split || p.vec) {
+      if (m >= p.M) return;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int n = nw + 8 * q + 4 * half;
+        const float fe[4] = {v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
+        if (split || !p.y_bf16) {
+          float *dst = split ? part + (size_t)m * p.part_N + n
+                             : reinterpret_cast<float *>(mat.y) + (size_t)m * mat.y_stride + n;
+          if (n + 4 <= (split ? (N + 3) & ~3 : N)) {
+            *reinterpret_cast<float4 *>(dst) = make_float4(fe[0], fe[1], fe[2], fe[3]);
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              if (n + e < N) dst[e] = fe[e];
+          }
+        } else {
+          __bf16 *dst = reinterpret_cast<__bf16 *>(mat.y) + (size_t)m * mat.y_stride + n;
+          if (n + 4 <= N) {
+            typedef __bf16 b4 __attribute__((ext_vector_type(4)));
+            *reinterpret_cast<b4 *>(dst) = b4{(__bf16)fe[0], (__bf16)fe[1], (__bf16)fe[2], (__bf16)fe[3]};
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              if (n + e < N) dst[e] = (__bf16)fe[e];
+          }
+        }
+      }
+    } else {
+      // rows off 16 bytes: element stores of 32 consecutive columns, the tile
+      // turned through LDS
+#pragma unroll
+      for (int e = 0; e < 16; ++e) flat[l32 * 33 + 8 * (e / 4) + 4 * half + e % 4] = v[e];
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int row = 2 * e + half, mm = bm0 + 32 * i + row, n = nw + l32;
+        const float f = flat[row * 33 + l32];
+        if (mm < p.M && n < N) {
+          if (p.y_bf16) reinterpret_cast<__bf16 *>(mat.y)[(size_t)mm * mat.y_stride + n] = (__bf16)f;
+          else reinterpret_cast<float *>(mat.y)[(size_t)mm * mat.y_stride + n] = f;
+        }
+      }
+    }
+  };
+  // a round: the tiles 2 r and 2 r + 1; each wave hands over the one it does not own
+  float4 *const mine = reinterpret_cast<float4 *>(smem + wave * 4096) + lane;
+  const float4 *const other = reinterpret_cast<const float4 *>(smem + (wave ^ 4) * 4096) + lane;
+#pragma unroll
+  for (int r = 0; r < (MI + 1) / 2; ++r) {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __syncthreads();  // the stages (or the last round's sums) are read
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      if (2 * r + q < MI && kg != q) {
+        const f32x16 &v = acc[2 * r + q < MI ? 2 * r + q : 0];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) mine[64 * c] = make_float4(v[4 * c], v[4 * c + 1], v[4 * c + 2], v[4 * c + 3]);
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      if (2 * r + q < MI && kg == q) {
+        f32x16 v = acc[2 * r + q < MI ? 2 * r + q : 0];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          const float4 f = other[64 * c];
+          v[4 * c] += f.x;
+          v[4 * c + 1] += f.y;
+          v[4 * c + 2] += f.z;
+          v[4 * c + 3] += f.w;
+        }
+        store(2 * r + q, v);
+      }
+    }
+  }
+}
+
 // sums the KS partial slices of a split product in k order (z = 0, 1, ...):
-// all KS loads of a thread are issued before the first add. V = 4: a thread
-// takes 4 consecutive columns of one row with 16-byte loads (partial rows and
-// every matrix's first column a multiple of 4 columns, vec bit 1), so the 4
-// never cross a matrix or a row; the y store is then one 8- or 16-byte store
-// when y rows are 16-byte aligned (vec bit 0).
-template <int KS, int V>
+// all KS loads of a thread are issued before the first add. A thread takes 4
+// consecutive columns of one row with 16-byte loads (every matrix's first
+// column and the rows are multiples of 4 columns: the 4 never cross a matrix
+// or a row, and only a matrix's last may lie past its end); the y store is
+// then one 8- or 16-byte store when y rows are 16-byte aligned.
+template <int KS>
 __global__ __launch_bounds__(256) void qmm_reduce_multi_kernel(QmmMulti p, int slot) {
-  typedef float fv __attribute__((ext_vector_type(V)));
+  typedef float fv __attribute__((ext_vector_type(4)));
   const float *part = g_qmm_part + (size_t)slot * kQSlotFloats;
-  const size_t MN = (size_t)p.M * p.part_N, nv = MN / V;
+  const size_t MN = (size_t)p.M * p.part_N, nv = MN / 4;
   for (size_t v = (size_t)blockIdx.x * 256 + threadIdx.x; v < nv; v += (size_t)gridDim.x * 256) {
-    const size_t i = v * V;
+    const size_t i = v * 4;
     fv t[KS];
 #pragma unroll
     for (int z = 0; z < KS; ++z) t[z] = __builtin_nontemporal_load(reinterpret_cast<const fv *>(part + z * MN + i));
@@ -514,494 +785,42 @@ __global__ __launch_bounds__(256) void qmm_reduce_multi_kernel(QmmMulti p, int s
 #pragma unroll
     for (int u = 1; u < kQMultiMax; ++u) mi = u < p.n && c >= p.m[u].col0 ? u : mi;
     const QmmMat &q = p.m[mi];
-    const size_t o = (size_t)m * q.y_stride + (c - q.col0);
+    const int n = c - q.col0;
+    const size_t o = (size_t)m * q.y_stride + n;
+    const bool vec = p.vec && n + 4 <= q.N;
     if (p.y_bf16) {
       __bf16 *y = reinterpret_cast<__bf16 *>(q.y) + o;
-      if constexpr (V == 4) {
-        if (p.vec & 1) {
-          typedef __bf16 b4 __attribute__((ext_vector_type(4)));
-          *reinterpret_cast<b4 *>(y) = b4{(__bf16)s[0], (__bf16)s[1], (__bf16)s[2], (__bf16)s[3]};
-          continue;
-        }
+      if (vec) {
+        typedef __bf16 b4 __attribute__((ext_vector_type(4)));
+        *reinterpret_cast<b4 *>(y) = b4{(__bf16)s[0], (__bf16)s[1], (__bf16)s[2], (__bf16)s[3]};
+        continue;
       }
 #pragma unroll
-      for (int e = 0; e < V; ++e) y[e] = (__bf16)s[e];
+      for (int e = 0; e < 4; ++e)
+        if (n + e < q.N) y[e] = (__bf16)s[e];
     } else {
       float *y = reinterpret_cast<float *>(q.y) + o;
-      if constexpr (V == 4) {
-        if (p.vec & 1) {
-          *reinterpret_cast<fv *>(y) = s;
-          continue;
-        }
+      if (vec) {
+        *reinterpret_cast<fv *>(y) = s;
+        continue;
       }
 #pragma unroll
-      for (int e = 0; e < V; ++e) y[e] = s[e];
+      for (int e = 0; e < 4; ++e)
+        if (n + e < q.N) y[e] = s[e];
     }
   }
 }
 
-template <int V>
 static void launch_qmm_reduce_multi(const QmmMulti &p, int slot, int KS, hipStream_t st) {
-  const size_t nv = (size_t)p.M * p.part_N / V;
+  const size_t nv = (size_t)p.M * p.part_N / 4;
   const dim3 grid((unsigned)std::min<size_t>((nv + 255) / 256, 4096));
   switch (KS) {
 #define LH_QRED(k) \
-  case k: hipLaunchKernelGGL((qmm_reduce_multi_kernel<k, V>), grid, dim3(256), 0, st, p, slot); break;
+  case k: hipLaunchKernelGGL((qmm_reduce_multi_kernel<k>), grid, dim3(256), 0, st, p, slot); break;
     LH_QRED(2) LH_QRED(3) LH_QRED(4) LH_QRED(5) LH_QRED(6) LH_QRED(7) LH_QRED(8) LH_QRED(9)
     LH_QRED(10) LH_QRED(11) LH_QRED(12) LH_QRED(13) LH_QRED(14) LH_QRED(15) LH_QRED(16)
 #undef LH_QRED
     default: break;
-  }
-}
-
-template <int BITS>
-__global__ __launch_bounds__(512) void affine_qmm256_kernel(QmmMulti p, int mtiles, int ntiles,
-                                                            int ksteps, int slot) {
-  __shared__ __align__(16) uint16_t sX[2][kQ3M * kQ3Ld];
-  __shared__ __align__(16) uint16_t sW[2][kQ3N * kQ3Ld];
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave >> 1, wn = wave & 1;
-  const int half = lane >> 5, l32 = lane & 31;
-  // XCD-grouped tile order: the M tiles of one N tile share an XCD's L2
-  const int L = blockIdx.x;
-  const int grp = L / (8 * mtiles), rem = L % (8 * mtiles);
-  const int nt = grp * 8 + rem % 8, mt = rem / 8;
-  if (nt >= ntiles) return;
-  int mi = 0;
-#pragma unroll
-  for (int t = 1; t < kQMultiMax; ++t) mi = t < p.n && nt >= p.tile_start[t] ? t : mi;
-  mi = __builtin_amdgcn_readfirstlane(mi);
-  const QmmMat &mat = p.m[mi];
-  const int bm0 = mt * kQ3M, bn0 = (nt - p.tile_start[mi]) * kQ3N;
-  const int N = mat.N;
-
-  // dequantising role: row wr of the W tile, codes [16 q, 16 q + 16) of each step
-  const int wr = tid >> 2, q = tid & 3;
-  const int nrow = min(bn0 + wr, N - 1);
-  const __amdgpu_buffer_rsrc_t wrs = q3_rsrc(mat.w, (long long)N * mat.row_bytes);
-  const __amdgpu_buffer_rsrc_t srs = q3_rsrc(mat.sc, (long long)N * mat.ng * 2);
-  const __amdgpu_buffer_rsrc_t brs = q3_rsrc(mat.bi, (long long)N * mat.ng * 2);
-  const int rowoff = (int)((long long)nrow * mat.row_bytes);
-  const int prow = nrow * mat.ng;
-  const int gsh = __builtin_ctz(p.gs);  // group sizes are powers of two here
-  const int sh5 = (BITS == 5 && (q & 1)) ? 16 : 0;  // 5-bit run start inside its first dword
-  const int wdst = wr * kQ3Ld;
-
-  // x staging role: 16-byte granules g = 512 i + tid (i < 4) of the 256 x 8
-  // tile
-  const uint16_t *xsrc[4];
-  int xdst[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int g = 512 * i + tid;
-    const int r = g >> 3, lg = g & 7;
-    xsrc[i] = p.x + (size_t)min(bm0 + r, p.M - 1) * p.x_stride + 8 * lg;
-    xdst[i] = r * kQ3Ld + 8 * lg;
-  }
-
-  const int z = blockIdx.y;
-  const int kb = z * ksteps * 64;
-  const int nst = (min(p.K, kb + ksteps * 64) - kb) >> 6;
-
-  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-  struct Set {
-    u32x4 x[4];  // native vectors: a HIP uint4 array copy would stay in memory
-    Q3Raw<BITS> w;
-  };
-  auto load = [&](int s, Set &r) {
-    const int k0 = kb + 64 * s;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) r.x[i] = *reinterpret_cast<const u32x4 *>(xsrc[i] + k0);
-    const int k = k0 + 16 * q;
-    q3_load<BITS>(r.w, wrs, srs, brs, rowoff, 2 * (prow + (k >> gsh)), k);
-  };
-  auto stage = [&](const Set &r, int st) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) *reinterpret_cast<u32x4 *>(sX[st] + xdst[i]) = r.x[i];
-    uint32_t pk[8];
-    q3_dequant<BITS>(r.w, sh5, p.fp16 != 0, pk);
-    uint16_t *d = sW[st] + wdst;
-    *reinterpret_cast<uint4 *>(d + 16 * q) = make_uint4(pk[0], pk[1], pk[2], pk[3]);
-    *reinterpret_cast<uint4 *>(d + 16 * q + 8) = make_uint4(pk[4], pk[5], pk[6], pk[7]);
-  };
-
-  f32x16 acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = f32x16{};
-  auto mfma = [&](int st) {
-    const uint16_t *xa = sX[st] + (wm * 64 + l32) * kQ3Ld;
-    const uint16_t *wb = sW[st] + (wn * 64 + l32) * kQ3Ld;
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      const int g = 16 * ks + 8 * half;
-      bf16x8 a[2], b[2];
-#pragma unroll
-      for (int i = 0; i < 2; ++i) a[i] = *reinterpret_cast<const bf16x8 *>(xa + 32 * kQ3Ld * i + g);
-#pragma unroll
-      for (int j = 0; j < 2; ++j) b[j] = *reinterpret_cast<const bf16x8 *>(wb + 32 * kQ3Ld * j + g);
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
-    }
-  };
-  auto barrier = [&]() {
-    // nothing moves across a step boundary (the scheduler would otherwise
-    // hoist the next set's conversions and wait for loads meant to stay in
-    // flight); the LDS writes of this wave are done, then the barrier alone
-    __builtin_amdgcn_sched_barrier(0);
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_sched_barrier(0);
-  };
-
-  // Step s's x and W pass through a register set loaded two steps earlier,
-  // are written (W dequantised) into LDS stage s & 1 one step ahead, and
-  // multiplied after the barrier that follows. Iteration s: barrier; the
-  // MFMAs of step s (they run in the matrix pipe while the same wave goes
-  // on); stage step s + 1 from its set into the other stage; load step s + 3
-  // into that set.
-  Set ra, rb;
-  load(0, ra);
-  if (nst > 1) load(1, rb);
-  stage(ra, 0);
-  if (nst > 2) load(2, ra);
-  int s = 0;
-  // steady state, two steps per trip so each register set is a fixed one
-  for (; s + 4 < nst; s += 2) {
-    barrier();
-    mfma(0);
-    stage(rb, 1);
-    load(s + 3, rb);
-    barrier();
-    mfma(1);
-    stage(ra, 0);
-    load(s + 4, ra);
-  }
-  // tail: the last (at most four) steps, s even here; written out so that
-  // each register set stays a fixed one
-  if (s < nst) {
-    barrier();
-    mfma(0);
-    if (s + 1 < nst) stage(rb, 1);
-    if (s + 3 < nst) load(s + 3, rb);
-  }
-  if (s + 1 < nst) {
-    barrier();
-    mfma(1);
-    if (s + 2 < nst) stage(ra, 0);
-    if (s + 4 < nst) load(s + 4, ra);
-  }
-  if (s + 2 < nst) {
-    barrier();
-    mfma(0);
-    if (s + 3 < nst) stage(rb, 1);
-  }
-  if (s + 3 < nst) {
-    barrier();
-    mfma(1);
-  }
-
-  // Output through LDS, 32 rows of the wave's tile at a time: the wave
-  // writes them as f32 rows of 72 floats (element e of MFMA tile (i, j) is
-  // row 8 (e / 4) + 4 half + e % 4, column 32 j + l32), then stores whole
-  // rows with 16-byte stores (8 bf16 or 4 f32 per lane); ragged or unaligned
-  // edges take element stores.
-  constexpr int kTs = 72;
-  __builtin_amdgcn_sched_barrier(0);
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  __builtin_amdgcn_s_barrier();  // every wave is done with the operand tiles
-  float *tb = reinterpret_cast<float *>(&sX[0][0]) + wave * (32 * kTs);
-  const bool split = slot >= 0;
-  float *part = split ? g_qmm_part + (size_t)slot * kQSlotFloats + (size_t)z * p.M * p.part_N + mat.col0
-                      : nullptr;
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e)
-        tb[(8 * (e / 4) + 4 * half + (e % 4)) * kTs + 32 * j + l32] = acc[i][j][e];
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_wave_barrier();
-    const int m0 = bm0 + wm * 64 + 32 * i, n0 = bn0 + wn * 64;
-    if (!split && p.y_bf16) {
-#pragma unroll
-      for (int it = 0; it < 4; ++it) {
-        const int r = 8 * it + (lane >> 3), c = 8 * (lane & 7);
-        const float4 u = *reinterpret_cast<const float4 *>(tb + r * kTs + c);
-        const float4 v = *reinterpret_cast<const float4 *>(tb + r * kTs + c + 4);
-        const int m = m0 + r, n = n0 + c;
-        if (m >= p.M) continue;
-        __bf16 *dst = reinterpret_cast<__bf16 *>(mat.y) + (size_t)m * mat.y_stride + n;
-        const float f[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
-        if ((p.vec & 1) && n + 8 <= N) {
-          bf16x8 o;
-#pragma unroll
-          for (int t = 0; t < 8; ++t) o[t] = (__bf16)f[t];
-          *reinterpret_cast<bf16x8 *>(dst) = o;
-        } else {
-#pragma unroll
-          for (int t = 0; t < 8; ++t)
-            if (n + t < N) dst[t] = (__bf16)f[t];
-        }
-      }
-    } else {
-      const bool vec = split ? (p.vec & 2) != 0 : (p.vec & 1) != 0;
-#pragma unroll
-      for (int it = 0; it < 8; ++it) {
-        const int r = 4 * it + (lane >> 4), c = 4 * (lane & 15);
-        const float4 u = *reinterpret_cast<const float4 *>(tb + r * kTs + c);
-        const int m = m0 + r, n = n0 + c;
-        if (m >= p.M) continue;
-        float *dst = split ? part + (size_t)m * p.part_N + n
-                           : reinterpret_cast<float *>(mat.y) + (size_t)m * mat.y_stride + n;
-        if (vec && n + 4 <= N) {
-          *reinterpret_cast<float4 *>(dst) = u;
-        } else {
-          const float f[4] = {u.x, u.y, u.z, u.w};
-#pragma unroll
-          for (int t = 0; t < 4; ++t)
-            if (n + t < N) dst[t] = f[t];
-        }
-      }
-    }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_wave_barrier();
-  }
-}
-
-// ---------------------------------------------------------------------------
-// The same 256 x 128 tiles with 16 waves (1024 threads): waves 8 (m) x 2 (n),
-// each a 32 x 64 tile (1 x 2 v_mfma_f32_32x32x16_bf16 tiles), each thread
-// dequantising 8 codes and staging 2 granules of x per step. Same LDS layout,
-// tile order and one-barrier-per-step pipeline as affine_qmm256_kernel, at
-// <= 128 registers so that four waves share a SIMD instead of two: the step's
-// chain of LDS reads -> MFMAs and loads -> dequantisation -> LDS writes ->
-// barrier then overlaps across twice the waves.
-template <int BITS>
-struct Q8Raw {
-  uint32_t w[BITS == 4 ? 1 : 2];
-  uint32_t s, b;
-};
-
-// 8 codes [k, k + 8) of a row (k a multiple of 8) and their group's scale
-// and bias
-template <int BITS>
-__device__ __forceinline__ void q8_load(Q8Raw<BITS> &r, __amdgpu_buffer_rsrc_t wr,
-                                        __amdgpu_buffer_rsrc_t sr, __amdgpu_buffer_rsrc_t br,
-                                        int rowoff, int poff, int k) {
-  if constexpr (BITS == 4) {
-    r.w[0] = __builtin_amdgcn_raw_buffer_load_b32(wr, rowoff + (k >> 1), 0, 0);
-  } else if constexpr (BITS == 8) {
-    const uint2 v = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(wr, rowoff + k, 0, 0));
-    r.w[0] = v.x;
-    r.w[1] = v.y;
-  } else {
-    // the dword holding the first code; the 8 codes end within the next one
-    const uint2 v = __builtin_bit_cast(
-        uint2, __builtin_amdgcn_raw_buffer_load_b64(wr, rowoff + 4 * ((k * BITS) >> 5), 0, 0));
-    r.w[0] = v.x;
-    r.w[1] = v.y;
-  }
-  r.s = __builtin_amdgcn_raw_buffer_load_b16(sr, poff, 0, 0);
-  r.b = __builtin_amdgcn_raw_buffer_load_b16(br, poff, 0, 0);
-}
-
-// bf16(code * s + b) of the 8 codes, packed in pairs (code order); sh is the
-// bit of the first code within r.w[0] (5/6-bit)
-template <int BITS>
-__device__ __forceinline__ void q8_dequant(const Q8Raw<BITS> &r, int sh, bool fp16, uint32_t (&pk)[4]) {
-  const float s = aux_to_f32_sel(r.s, fp16), b = aux_to_f32_sel(r.b, fp16);
-  float f[8];
-  if constexpr (BITS == 4) {
-    const uint32_t lo = r.w[0] & 0x0F0F0F0Fu, hi = (r.w[0] >> 4) & 0x0F0F0F0Fu;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      f[2 * i] = (float)((lo >> (8 * i)) & 255u);
-      f[2 * i + 1] = (float)((hi >> (8 * i)) & 255u);
-    }
-  } else if constexpr (BITS == 8) {
-#pragma unroll
-    for (int d = 0; d < 2; ++d)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) f[4 * d + i] = (float)((r.w[d] >> (8 * i)) & 255u);
-  } else {
-    const uint32_t win[2] = {__builtin_amdgcn_alignbit(r.w[1], r.w[0], sh), r.w[1] >> sh};
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int bit = j * BITS, i = bit >> 5, o = bit & 31;
-      uint32_t v = win[i] >> o;
-      if (o + BITS > 32) v |= win[i + 1] << (32 - o);
-      f[j] = (float)(v & ((1u << BITS) - 1u));
-    }
-  }
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    bf16x2 v;
-    v[0] = (__bf16)fmaf(f[2 * j], s, b);
-    v[1] = (__bf16)fmaf(f[2 * j + 1], s, b);
-    pk[j] = __builtin_bit_cast(uint32_t, v);
-  }
-}
-
-template <int BITS>
-__global__ __launch_bounds__(1024) void affine_qmm256w_kernel(QmmMulti p, int mtiles, int ntiles,
-                                                              int ksteps, int slot) {
-  __shared__ __align__(16) uint16_t sX[2][kQ3M * kQ3Ld];
-  __shared__ __align__(16) uint16_t sW[2][kQ3N * kQ3Ld];
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave >> 1, wn = wave & 1;
-  const int half = lane >> 5, l32 = lane & 31;
-  const int L = blockIdx.x;
-  const int grp = L / (8 * mtiles), rem = L % (8 * mtiles);
-  const int nt = grp * 8 + rem % 8, mt = rem / 8;
-  if (nt >= ntiles) return;
-  int mi = 0;
-#pragma unroll
-  for (int t = 1; t < kQMultiMax; ++t) mi = t < p.n && nt >= p.tile_start[t] ? t : mi;
-  mi = __builtin_amdgcn_readfirstlane(mi);
-  const QmmMat &mat = p.m[mi];
-  const int bm0 = mt * kQ3M, bn0 = (nt - p.tile_start[mi]) * kQ3N;
-  const int N = mat.N;
-
-  // dequantising role: row wr of the W tile, codes [8 q, 8 q + 8) of each step
-  const int wr = tid >> 3, q = tid & 7;
-  const int nrow = min(bn0 + wr, N - 1);
-  const __amdgpu_buffer_rsrc_t wrs = q3_rsrc(mat.w, (long long)N * mat.row_bytes);
-  const __amdgpu_buffer_rsrc_t srs = q3_rsrc(mat.sc, (long long)N * mat.ng * 2);
-  const __amdgpu_buffer_rsrc_t brs = q3_rsrc(mat.bi, (long long)N * mat.ng * 2);
-  const int rowoff = (int)((long long)nrow * mat.row_bytes);
-  const int prow = nrow * mat.ng;
-  const int gsh = __builtin_ctz(p.gs);
-  // first code's bit within its dword: (8 q * BITS) mod 32 (k0 is a multiple of 64)
-  const int shq = (8 * q * BITS) & 31;
-  const int wdst = wr * kQ3Ld + 8 * q;
-
-  // x staging role: 16-byte granules g = 1024 i + tid (i < 2) of the 256 x 8 tile
-  const uint16_t *xsrc[2];
-  int xdst[2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int g = 1024 * i + tid;
-    const int r = g >> 3, lg = g & 7;
-    xsrc[i] = p.x + (size_t)min(bm0 + r, p.M - 1) * p.x_stride + 8 * lg;
-    xdst[i] = r * kQ3Ld + 8 * lg;
-  }
-
-  const int z = blockIdx.y;
-  const int kb = z * ksteps * 64;
-  const int nst = (min(p.K, kb + ksteps * 64) - kb) >> 6;
-
-  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-  struct Set {
-    u32x4 x[2];
-    Q8Raw<BITS> w;
-  };
-  auto load = [&](int s, Set &r) {
-    const int k0 = kb + 64 * s;
-#pragma unroll
-    for (int i = 0; i < 2; ++i) r.x[i] = *reinterpret_cast<const u32x4 *>(xsrc[i] + k0);
-    const int k = k0 + 8 * q;
-    q8_load<BITS>(r.w, wrs, srs, brs, rowoff, 2 * (prow + (k >> gsh)), k);
-  };
-  auto stage = [&](const Set &r, int st) {
-#pragma unroll
-    for (int i = 0; i < 2; ++i) *reinterpret_cast<u32x4 *>(sX[st] + xdst[i]) = r.x[i];
-    uint32_t pk[4];
-    q8_dequant<BITS>(r.w, shq, p.fp16 != 0, pk);
-    *reinterpret_cast<uint4 *>(sW[st] + wdst) = make_uint4(pk[0], pk[1], pk[2], pk[3]);
-  };
-
-  f32x16 acc[2];
-#pragma unroll
-  for (int j = 0; j < 2; ++j) acc[j] = f32x16{};
-  auto mfma = [&](int st) {
-    const uint16_t *xa = sX[st] + (wm * 32 + l32) * kQ3Ld;
-    const uint16_t *wb = sW[st] + (wn * 64 + l32) * kQ3Ld;
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      const int g = 16 * ks + 8 * half;
-      const bf16x8 a = *reinterpret_cast<const bf16x8 *>(xa + g);
-      bf16x8 b[2];
-#pragma unroll
-      for (int j = 0; j < 2; ++j) b[j] = *reinterpret_cast<const bf16x8 *>(wb + 32 * kQ3Ld * j + g);
-#pragma unroll
-      for (int j = 0; j < 2; ++j) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b[j], acc[j], 0, 0, 0);
-    }
-  };
-  auto barrier = [&]() {
-    __builtin_amdgcn_sched_barrier(0);
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_sched_barrier(0);
-  };
-
-  // as affine_qmm256_kernel: step s's operands pass through a register set
-  // loaded two steps earlier and LDS stage s & 1 written one step ahead
-  Set ra, rb;
-  load(0, ra);
-  if (nst > 1) load(1, rb);
-  stage(ra, 0);
-  if (nst > 2) load(2, ra);
-  int s = 0;
-  for (; s + 4 < nst; s += 2) {
-    barrier();
-    mfma(0);
-    stage(rb, 1);
-    load(s + 3, rb);
-    barrier();
-    mfma(1);
-    stage(ra, 0);
-    load(s + 4, ra);
-  }
-  if (s < nst) {
-    barrier();
-    mfma(0);
-    if (s + 1 < nst) stage(rb, 1);
-    if (s + 3 < nst) load(s + 3, rb);
-  }
-  if (s + 1 < nst) {
-    barrier();
-    mfma(1);
-    if (s + 2 < nst) stage(ra, 0);
-    if (s + 4 < nst) load(s + 4, ra);
-  }
-  if (s + 2 < nst) {
-    barrier();
-    mfma(0);
-    if (s + 3 < nst) stage(rb, 1);
-  }
-  if (s + 3 < nst) {
-    barrier();
-    mfma(1);
-  }
-
-  // element e of tile j: row 8 (e / 4) + 4 half + e % 4 of the wave's 32,
-  // column 32 j + l32 of its 64; lanes 0-31 store 32 consecutive columns
-  const bool split = slot >= 0;
-  float *part = split ? g_qmm_part + (size_t)slot * kQSlotFloats + (size_t)z * p.M * p.part_N + mat.col0
-                      : nullptr;
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int n = bn0 + wn * 64 + 32 * j + l32;
-    if (n >= N) continue;
-#pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      const int m = bm0 + wm * 32 + 8 * (e / 4) + 4 * half + (e % 4);
-      if (m >= p.M) continue;
-      if (split)
-        part[(size_t)m * p.part_N + n] = acc[j][e];
-      else if (p.y_bf16)
-        reinterpret_cast<__bf16 *>(mat.y)[(size_t)m * mat.y_stride + n] = (__bf16)acc[j][e];
-      else
-        reinterpret_cast<float *>(mat.y)[(size_t)m * mat.y_stride + n] = acc[j][e];
-    }
   }
 }
 
@@ -1014,27 +833,75 @@ bool affine_qmm_supported(const DevMat &m) {
   return true;
 }
 
-// 256 x 128 tiles: every matrix supported, the same K / bits / group size /
-// aux type, power-of-two group sizes (the kernel shifts), at least 256 rows
-// of x, and offsets of every matrix within 2 GiB (32-bit buffer offsets)
-static bool qmm256_ok(const DevMat *ms, int n, int M) {
-  if (M < kQ3M || n < 1 || n > kQMultiMax) return false;
+// The tile kernel: every matrix supported, the same K / bits / group size /
+// aux type, 16-byte copies of the packed rows (5-bit rows: 4-byte ones) and
+// per-lane offsets within a tile that fit 32 bits.
+static bool qmm_tile_ok(const DevMat *ms, int n, int x_stride) {
+  if (n < 1 || n > kQMultiMax || x_stride > (1 << 22)) return false;
   for (int i = 0; i < n; ++i) {
     const DevMat &m = ms[i];
     if (!affine_qmm_supported(m)) return false;
     if (m.I != ms[0].I || m.bits != ms[0].bits || m.gs != ms[0].gs || m.fp16 != ms[0].fp16) return false;
-    if ((m.gs & (m.gs - 1)) != 0 || (long long)m.O * m.row_bytes > 0x7fffffffLL) return false;
-    if ((reinterpret_cast<uintptr_t>(m.w) & 15) != 0) return false;
+    if (m.bits != 5 && (reinterpret_cast<uintptr_t>(m.w) & 15) != 0) return false;
+    if (m.row_bytes > (1 << 23) || (long long)m.O * m.ng > 0x7fff0000LL / 2) return false;
+    // scale / bias rows are copied by dwords
+    if (((reinterpret_cast<uintptr_t>(m.sc) | reinterpret_cast<uintptr_t>(m.bi)) & 3) != 0) return false;
+    if ((long long)m.O * m.ng < 2) return false;
   }
   return true;
 }
 
-// 16 waves per block where K is split (short k ranges: the 2048-row output
-// projections, 23 -> 19.6 us), 8 where it is not (the 12352-row grids of one
-// k range, 45.4 -> 43 us)
+// Tile rows and K split of a product: the least estimated time in us. The
+// constants are fitted to 1,450 measured (M, N, K, bits, rows, split) between
+// 24 and 2048 rows, 1024 and 28672 columns (mean error 6 %; the choice costs
+// 0.2 % over the best one measured): a 64-k step of a block, whose weights
+// are formed whatever its rows, or the time its codes take to arrive; a
+// block's pipeline fill and sum exchange; and for a split its partial sums
+// written and read back and one more launch. One block per CU.
+struct QmmPlan {
+  int bm, split;
+};
+static QmmPlan qmm_plan(int M, int tiles, int cols, int ksteps, int bits) {
+  static const int kBm[5] = {32, 64, 128, 192, 256};
+  QmmPlan best{256, 1};
+  float tb = 1e30f;
+  for (int c = 0; c < 5; ++c) {
+    const int bm = kBm[c], mt = (M + bm - 1) / bm;
+    const float step = std::max(0.39f + 0.32f * bm / 256, 0.33f * bits / 8);
+    const float fixed = 1.8f + 5.0f * bm / 256;
+    for (int sp = 1; sp <= 16; ++sp) {
+      const int ks = (ksteps + sp - 1) / sp;
+      if ((ksteps + ks - 1) / ks != sp) continue;
+      if (sp > 1 && (ks < 3 || (size_t)sp * M * cols > kQSlotFloats)) continue;
+      const int rounds = (int)(((long long)mt * tiles * sp + 255) / 256);
+      float t = rounds * (ks * step + fixed);
+      if (sp > 1) t += 4.4f + (float)sp * M * cols * 8 / 5.5e6f;
+      if (t < tb) {
+        tb = t;
+        best = QmmPlan{bm, sp};
+      }
+    }
+  }
+  return best;
+}
 
-static hipError_t launch_qmm256(const DevMat *ms, int n, const uint16_t *x, int x_stride, int M,
-                                void *const *ys, const int *y_strides, int y_bf16, hipStream_t st) {
+template <int BITS, bool GS64, bool FP16>
+static hipError_t launch_qmm_tile_bits(const QmmMulti &p, int bm, int mt, int tiles, int split, int ksteps,
+                                       int slot, hipStream_t st) {
+  const dim3 grid((mt * tiles * split + 7) / 8 * 8), block(512);
+  switch (bm) {
+#define LH_QTILE(MI)                                                                                      \
+  case 32 * MI: hipLaunchKernelGGL((affine_qmm_tile_kernel<BITS, MI, GS64, FP16>), grid, block, 0, st, p, \
+                                   mt, tiles, ksteps, slot); break;
+    LH_QTILE(1) LH_QTILE(2) LH_QTILE(4) LH_QTILE(6) LH_QTILE(8)
+#undef LH_QTILE
+    default: return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
+}
+
+static hipError_t launch_qmm_tile(const DevMat *ms, int n, const uint16_t *x, int x_stride, int M,
+                                  void *const *ys, const int *y_strides, int y_bf16, hipStream_t st) {
   QmmMulti p;
   p.x = x;
   p.n = n;
@@ -1050,8 +917,8 @@ static hipError_t launch_qmm256(const DevMat *ms, int n, const uint16_t *x, int 
       p.m[i] = QmmMat{ms[i].w, ms[i].sc, ms[i].bi, ys[i], ms[i].row_bytes, ms[i].O, ms[i].ng,
                       y_strides[i], cols};
       p.tile_start[i] = tiles;
-      tiles += (ms[i].O + kQ3N - 1) / kQ3N;
-      cols += ms[i].O;
+      tiles += (ms[i].O + kTN - 1) / kTN;
+      cols += (ms[i].O + 3) & ~3;  // 16-byte partial stores
     } else {
       p.m[i] = p.m[0];
       p.tile_start[i] = tiles;
@@ -1059,53 +926,38 @@ static hipError_t launch_qmm256(const DevMat *ms, int n, const uint16_t *x, int 
   }
   p.tile_start[kQMultiMax] = tiles;
   p.part_N = cols;
-  bool yv = true, pv = (cols & 3) == 0;
+  bool yv = true;
   for (int i = 0; i < n; ++i) {
     const int es = y_bf16 ? 2 : 4;
     yv = yv && (reinterpret_cast<uintptr_t>(ys[i]) & 15) == 0 && ((long long)y_strides[i] * es) % 16 == 0;
-    pv = pv && (p.m[i].col0 & 3) == 0;
   }
-  p.vec = (yv ? 1 : 0) | (pv ? 2 : 0);
-  const int mt = (M + kQ3M - 1) / kQ3M;
+  p.vec = yv ? 1 : 0;
   const int ksteps_all = p.K / 64;
-  // split K while the grid is short of one block per CU and each k range
-  // keeps at least 8 steps
-  int split = 1;
-  while (split < 16 && mt * tiles * split < 192 && ksteps_all / (2 * split) >= 8 &&
-         (size_t)(2 * split) * M * cols <= kQSlotFloats)
-    split *= 2;
-  const int ksteps = (ksteps_all + split - 1) / split;
-  split = (ksteps_all + ksteps - 1) / ksteps;
+  const QmmPlan plan = qmm_plan(M, tiles, cols, ksteps_all, ms[0].bits);
+  const int mt = (M + plan.bm - 1) / plan.bm;
+  const int ksteps = (ksteps_all + plan.split - 1) / plan.split;
+  const int split = plan.split;
   SlotRing::Lease lease;
   if (split > 1) {
     const hipError_t le = g_qmm_slots.take(st, lease);
     if (le != hipSuccess) return le;
   }
   const int slot = split > 1 ? lease.slot() : -1;
-  const dim3 grid(((tiles + 7) / 8) * 8 * mt, split);
-  if (split > 1) {
-    switch (ms[0].bits) {
-      case 4: hipLaunchKernelGGL(affine_qmm256w_kernel<4>, grid, dim3(1024), 0, st, p, mt, tiles, ksteps, slot); break;
-      case 5: hipLaunchKernelGGL(affine_qmm256w_kernel<5>, grid, dim3(1024), 0, st, p, mt, tiles, ksteps, slot); break;
-      case 6: hipLaunchKernelGGL(affine_qmm256w_kernel<6>, grid, dim3(1024), 0, st, p, mt, tiles, ksteps, slot); break;
-      case 8: hipLaunchKernelGGL(affine_qmm256w_kernel<8>, grid, dim3(1024), 0, st, p, mt, tiles, ksteps, slot); break;
-      default: return hipErrorInvalidValue;
-    }
-  } else {
-    switch (ms[0].bits) {
-      case 4: hipLaunchKernelGGL(affine_qmm256_kernel<4>, grid, dim3(512), 0, st, p, mt, tiles, ksteps, slot); break;
-      case 5: hipLaunchKernelGGL(affine_qmm256_kernel<5>, grid, dim3(512), 0, st, p, mt, tiles, ksteps, slot); break;
-      case 6: hipLaunchKernelGGL(affine_qmm256_kernel<6>, grid, dim3(512), 0, st, p, mt, tiles, ksteps, slot); break;
-      case 8: hipLaunchKernelGGL(affine_qmm256_kernel<8>, grid, dim3(512), 0, st, p, mt, tiles, ksteps, slot); break;
-      default: return hipErrorInvalidValue;
-    }
+  hipError_t e;
+  switch (ms[0].bits) {
+#define LH_QBITS(B)                                                                                     \
+  case B:                                                                                               \
+    e = p.gs == 64 ? (p.fp16 ? launch_qmm_tile_bits<B, true, true>(p, plan.bm, mt, tiles, split, ksteps, slot, st)     \
+                             : launch_qmm_tile_bits<B, true, false>(p, plan.bm, mt, tiles, split, ksteps, slot, st))   \
+                   : (p.fp16 ? launch_qmm_tile_bits<B, false, true>(p, plan.bm, mt, tiles, split, ksteps, slot, st)    \
+                             : launch_qmm_tile_bits<B, false, false>(p, plan.bm, mt, tiles, split, ksteps, slot, st)); \
+    break;
+    LH_QBITS(4) LH_QBITS(5) LH_QBITS(6) LH_QBITS(8)
+#undef LH_QBITS
+    default: return hipErrorInvalidValue;
   }
-  hipError_t e = hipGetLastError();
   if (e != hipSuccess || split == 1) return e;
-  if (p.vec & 2)
-    launch_qmm_reduce_multi<4>(p, slot, split, st);
-  else
-    launch_qmm_reduce_multi<1>(p, slot, split, st);
+  launch_qmm_reduce_multi(p, slot, split, st);
   e = hipGetLastError();
   const hipError_t le = lease.done();
   return e != hipSuccess ? e : le;
@@ -1117,7 +969,7 @@ hipError_t launch_affine_qmm_multi(const DevMat *ms, int n, const uint16_t *x, i
   if ((reinterpret_cast<uintptr_t>(x) & 15) != 0 || (x_stride & 7) != 0) return hipErrorInvalidValue;
   int strides[kQMultiMax];
   for (int i = 0; i < n; ++i) strides[i] = ms[i].O;
-  if (qmm256_ok(ms, n, M)) return launch_qmm256(ms, n, x, x_stride, M, ys, strides, y_bf16, st);
+  if (n > 1 && qmm_tile_ok(ms, n, x_stride)) return launch_qmm_tile(ms, n, x, x_stride, M, ys, strides, y_bf16, st);
   for (int i = 0; i < n; ++i) {
     const hipError_t e = launch_affine_qmm(ms[i], x, x_stride, M, ys[i], ms[i].O, y_bf16, st);
     if (e != hipSuccess) return e;
@@ -1128,12 +980,19 @@ hipError_t launch_affine_qmm_multi(const DevMat *ms, int n, const uint16_t *x, i
 hipError_t launch_affine_qmm(const DevMat &m, const uint16_t *x, int x_stride, int M, void *y,
                              int y_stride, int y_bf16, hipStream_t st) {
   if (!affine_qmm_supported(m) || M <= 0) return hipErrorInvalidValue;
-  if (qmm256_ok(&m, 1, M) && (reinterpret_cast<uintptr_t>(x) & 15) == 0 && (x_stride & 7) == 0) {
+  if ((reinterpret_cast<uintptr_t>(x) & 15) != 0 || (x_stride & 7) != 0) return hipErrorInvalidValue;
+  // Products this small are launch and latency: the tile kernel's prologue (its
+  // rings, three or more steps ahead) and sum exchange cost more than they
+  // save. us, 64 x 64 kernel / tile kernel, 4-bit: 17 x 512 (M x N), K 2048:
+  // 8.0 / 9.0; 17 x 4096, K 2048: 10.6 / 11.1; 64 x 1024, K 2048: 10.3 / 10.3;
+  // 64 x 2048, K 2048: 13.6 / 11.9; 17 x 1024, K 9728: 13.2 / 13.7;
+  // 17 x 2048, K 9728: 16.2 / 14.4.
+  const bool small = (long long)M * m.O <= (M <= 24 ? 81920 : 65536) && (long long)m.O * m.I <= (10 << 20);
+  if (!small && qmm_tile_ok(&m, 1, x_stride)) {
     void *ys[1] = {y};
     const int strides[1] = {y_stride};
-    return launch_qmm256(&m, 1, x, x_stride, M, ys, strides, y_bf16, st);
+    return launch_qmm_tile(&m, 1, x, x_stride, M, ys, strides, y_bf16, st);
   }
-  if ((reinterpret_cast<uintptr_t>(x) & 15) != 0 || (x_stride & 7) != 0) return hipErrorInvalidValue;
   GemmParams p;
   p.w = m.w;
   p.sc = m.sc;
@@ -1150,13 +1009,10 @@ hipError_t launch_affine_qmm(const DevMat &m, const uint16_t *x, int x_stride, i
   p.x_stride = x_stride;
   p.y_stride = y_stride;
   p.y_bf16 = y_bf16;
-  // Large tiles when their grid alone keeps the chip busy, else 64 x 64
-  // tiles (four times the blocks); grids still short of about two blocks per
-  // CU split K as well (at most 16 ways, partials within one slot).
+  // 64 x 64 tiles; grids short of about two blocks per CU split K as well (at
+  // most 16 ways, partials within one slot)
   const int ksteps_all = m.I / 64;
-  const int mt = (M + kQ2 - 1) / kQ2, nt = (m.O + kQ2 - 1) / kQ2;
-  const bool big = M > kTile && m.O >= kQ2 && (mt * nt >= kQ2MinTiles || m.I >= 512);
-  const int tiles = big ? mt * nt : ((M + kTile - 1) / kTile) * ((m.O + kTile - 1) / kTile);
+  const int tiles = ((M + kTile - 1) / kTile) * ((m.O + kTile - 1) / kTile);
   int split = 1;
   while (split < 16 && tiles * split < kQTargetBlocks && 2 * split <= ksteps_all &&
          (size_t)(2 * split) * M * m.O <= kQSlotFloats)
@@ -1169,22 +1025,12 @@ hipError_t launch_affine_qmm(const DevMat &m, const uint16_t *x, int x_stride, i
     if (le != hipSuccess) return le;
   }
   const int slot = split > 1 ? lease.slot() : -1;
-  if (big) {
-    const dim3 grid(((nt + 7) / 8) * 8 * mt, split);
-    switch (m.bits) {
-      case 4: hipLaunchKernelGGL(affine_qmm128_kernel<4>, grid, dim3(256), 0, st, p, mt, nt, ksteps, slot); break;
-      case 5: hipLaunchKernelGGL(affine_qmm128_kernel<5>, grid, dim3(256), 0, st, p, mt, nt, ksteps, slot); break;
-      case 6: hipLaunchKernelGGL(affine_qmm128_kernel<6>, grid, dim3(256), 0, st, p, mt, nt, ksteps, slot); break;
-      case 8: hipLaunchKernelGGL(affine_qmm128_kernel<8>, grid, dim3(256), 0, st, p, mt, nt, ksteps, slot); break;
-    }
-  } else {
-    const dim3 grid((M + kTile - 1) / kTile, (m.O + kTile - 1) / kTile, split);
-    switch (m.bits) {
-      case 4: hipLaunchKernelGGL(affine_qmm_kernel<4>, grid, dim3(256), 0, st, p, ksteps, slot); break;
-      case 5: hipLaunchKernelGGL(affine_qmm_kernel<5>, grid, dim3(256), 0, st, p, ksteps, slot); break;
-      case 6: hipLaunchKernelGGL(affine_qmm_kernel<6>, grid, dim3(256), 0, st, p, ksteps, slot); break;
-      case 8: hipLaunchKernelGGL(affine_qmm_kernel<8>, grid, dim3(256), 0, st, p, ksteps, slot); break;
-    }
+  const dim3 grid((M + kTile - 1) / kTile, (m.O + kTile - 1) / kTile, split);
+  switch (m.bits) {
+    case 4: hipLaunchKernelGGL(affine_qmm_kernel<4>, grid, dim3(256), 0, st, p, ksteps, slot); break;
+    case 5: hipLaunchKernelGGL(affine_qmm_kernel<5>, grid, dim3(256), 0, st, p, ksteps, slot); break;
+    case 6: hipLaunchKernelGGL(affine_qmm_kernel<6>, grid, dim3(256), 0, st, p, ksteps, slot); break;
+    case 8: hipLaunchKernelGGL(affine_qmm_kernel<8>, grid, dim3(256), 0, st, p, ksteps, slot); break;
   }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || split == 1) return e;

@@ -269,3 +269,50 @@ def test_split_qmm_on_three_overlapping_streams(gpu):
                                      sc.reshape(O, ng)[cols].reshape(-1),
                                      bi.reshape(O, ng)[cols].reshape(-1), len(cols), I, bits, gs)
         assert normwise_rel(serial[s].cpu().numpy()[:, cols], ref) <= 1e-5
+
+
+TILE_CASES = [
+    # (M, O, I, bits, gs, fp16): rows at the edges of the 32 / 64 / 128 / 192 /
+    # 256-row tiles; 1, 2, 3, 5, 9, 45 steps of 64 codes (pipelines that never
+    # fill, chunks of scale words that end early); rows of an odd number of
+    # groups, which start inside a dword; group sizes 32 to 192
+    (31, 130, 64, 8, 64, False),
+    (33, 257, 128, 4, 32, True),
+    (65, 96, 192, 6, 64, False),
+    (128, 384, 320, 5, 64, True),
+    (129, 200, 576, 8, 192, False),
+    (191, 132, 2880, 4, 64, False),
+    (193, 128, 384, 6, 96, True),
+    (256, 130, 448, 5, 32, False),
+    (257, 70, 832, 4, 64, True),
+    (513, 260, 1088, 8, 64, False),
+    # an odd total of groups: the last word is copied alone
+    (40, 33, 192, 4, 64, False),
+    (140, 161, 320, 8, 64, True),
+    # few column tiles: row tiles and k ranges in turn over the chip
+    (300, 64, 2048, 8, 128, False),
+]
+
+
+@pytest.mark.parametrize("M,O,I,bits,gs,fp16", TILE_CASES, ids=lambda v: str(v))
+def test_qmm_tile_edges(gpu, M, O, I, bits, gs, fp16):
+    """Every column against the oracle at shapes where tiles, pipelines and
+    scale rows end unevenly, weights at a 16-byte and at a 4-byte offset (the
+    64 x 64 kernel), the two within f32 rounding of each other."""
+    import torch
+    from logan_amd.device import AffineMatrix, affine_qmm
+
+    rng = np.random.default_rng(M * 7 + O + bits)
+    w, sc, bi = make_affine(rng, O, I, bits, gs, fp16)
+    xb = make_x(rng, M, I).reshape(M, I)
+    x = to_dev(xb.view(np.int16), torch).view(torch.bfloat16)
+    ref = oracle.affine_qmm_bf16(bf16_to_f32(xb).reshape(M, I), w, sc, bi, O, I, bits, gs, fp16)
+    m = dev_matrix(torch, w, sc, bi, O, I, bits, gs, fp16)
+    y = affine_qmm(m, x, out_dtype=torch.float32)
+    assert normwise_rel(y.cpu().numpy(), ref) <= 1e-5
+    buf = torch.empty(w.size + 16, dtype=torch.uint8, device="cuda")
+    off = buf[4:4 + w.size]
+    off.copy_(m.weights.reshape(-1))
+    m4 = AffineMatrix(off.view(m.weights.shape), m.scales, m.biases, O, I, bits, gs, fp16)
+    y4 = affine_qmm(m4, x, out_dtype=torch.float32)
+    assert normwise_rel(y4.cpu().numpy(), ref) <= 1e-5
