@@ -220,6 +220,34 @@ def test_device_llama_layer_config2_shape(gpu):
     assert torch.equal(xd5, xd)
 
 
+@pytest.mark.parametrize("H,KH,hd,pos", [(4, 2, 32, 511), (4, 2, 32, 512), (6, 2, 64, 33),
+                                         (16, 1, 32, 2053), (16, 2, 128, 1100)])
+def test_device_llama_layer_slice_joins(gpu, H, KH, hd, pos):
+    """Positions whose 32-position slices end on and past a batch of the join
+    (16 slices' o, 1024 / G slices' factors at a time), 1 to 16 query heads
+    per kv head: x, K and V against the oracle."""
+    import torch
+
+    from logan_amd.device import llama_layer
+
+    rng = np.random.default_rng(pos + H)
+    D, inter, theta, eps = 128, 256, 10000.0, 1e-5
+    mats = make_layer(rng, D, inter, H, KH, hd, (5,) * 7)
+    ones = np.ones(D, np.float32)
+    kc = rng.standard_normal((pos + 1, KH * hd)).astype(np.float32)
+    vc = rng.standard_normal((pos + 1, KH * hd)).astype(np.float32)
+    x = rng.standard_normal(D).astype(np.float32)
+    layer = _dev_layer(torch, mats, ones, ones, pos + 1, D, inter, H, KH, hd, theta, eps)
+    layer.k_cache.copy_(torch.from_numpy(kc))
+    layer.v_cache.copy_(torch.from_numpy(vc))
+    want = oracle.llama_layer(x, kc, vc, pos, mats, ones, ones, D, inter, H, KH, hd, theta, eps)
+    xd = torch.from_numpy(x).cuda()
+    llama_layer(layer, xd, pos)
+    assert rel(xd.cpu().numpy(), want) < TOL
+    assert rel(layer.k_cache[pos].cpu().numpy(), kc[pos]) < TOL
+    assert rel(layer.v_cache[pos].cpu().numpy(), vc[pos]) < TOL
+
+
 def test_device_llama_layer_rejects(gpu):
     import torch
 
