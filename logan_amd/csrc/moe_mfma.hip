@@ -18,6 +18,8 @@
 //      moe_gateup_lds_kernel   above 128 tokens (4/8-bit, groups of 64): the
 //                              weights streamed through a per-wave LDS ring,
 //                              whole-tile blocks and then 128-row ones
+//      moe_gateup_wide_kernel  the same over tiles of up to 64 slots, where an
+//                              expert has many (wide_tiles)
 //   4. moe_down_mfma_kernel    per (tile, 128 rows): h hi/lo staged in LDS,
 //                              two MFMA passes (hi, lo), y in grouped order
 //      moe_down_lds_kernel     above 128 tokens: the LDS ring again,
@@ -170,7 +172,7 @@ __global__ __launch_bounds__(256) void moe_mroute_kernel(MoeArgs a, MoeMWs w) {
 // ---------------------------------------------------------------------------
 // 2. grouping into tiles (one block)
 
-__global__ __launch_bounds__(kMGroupThreads) void moe_mgroup_kernel(MoeArgs a, MoeMWs w) {
+__global__ __launch_bounds__(kMGroupThreads) void moe_mgroup_kernel(MoeArgs a, MoeMWs w, int ts) {  // ts: slots per tile
   __shared__ int s_cnt[kMMaxE];
   __shared__ int s_start[kMMaxE];
   __shared__ int s_tbase[kMMaxE];
@@ -202,7 +204,7 @@ __global__ __launch_bounds__(kMGroupThreads) void moe_mgroup_kernel(MoeArgs a, M
     // tiles <= 2^12 + 2^10
     const int e = tid;
     const int c = e < a.E ? s_cnt[e] : 0;
-    const int v = (c << 14) | ((c + kMTok - 1) / kMTok);
+    const int v = (c << 14) | ((c + ts - 1) / ts);
     int incl = v;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
@@ -241,14 +243,14 @@ __global__ __launch_bounds__(kMGroupThreads) void moe_mgroup_kernel(MoeArgs a, M
   // the shared expert's tiles first, then the routed ones (the launches
   // give the first tiles whole-tile blocks)
   const int R = s_routed_tiles;
-  const int S = a.sgate.m.w ? (a.B + kMTok - 1) / kMTok : 0;
+  const int S = a.sgate.m.w ? (a.B + ts - 1) / ts : 0;
   for (int e = tid; e < a.E; e += kMGroupThreads) {
     const int c = s_cnt[e];
-    for (int tt = 0; tt * kMTok < c; ++tt)
-      w.tiles[S + s_tbase[e] + tt] = make_int4(e, s_start[e] + kMTok * tt, min(kMTok, c - kMTok * tt), 0);
+    for (int tt = 0; tt * ts < c; ++tt)
+      w.tiles[S + s_tbase[e] + tt] = make_int4(e, s_start[e] + ts * tt, min(ts, c - ts * tt), 0);
   }
   for (int tt = tid; tt < S; tt += kMGroupThreads)
-    w.tiles[tt] = make_int4(-1, nslots + kMTok * tt, min(kMTok, a.B - kMTok * tt), 0);
+    w.tiles[tt] = make_int4(-1, nslots + ts * tt, min(ts, a.B - ts * tt), 0);
   if (tid == 0) *w.n_tiles = R + S;
 }
 
@@ -791,6 +793,255 @@ __global__ __launch_bounds__(512, 1) void moe_gateup_lds_kernel(MoeArgs a, MoeMW
 }
 
 // ---------------------------------------------------------------------------
+// 3c. gate/up over tiles of up to 64 slots, for batches that give an expert
+//     more than one 16-slot tile. What bounds the 16-slot form there is that
+//     every tile of an expert streams and unpacks the expert's weights again
+//     (1999 tokens, 512 experts, top 10: 3 tiles an expert, 2 GB of codes into
+//     LDS for 0.6 GB of weights; unpacking is half of its vector work). Here a
+//     wave unpacks its 16 gate and 16 up rows once for up to four 16-slot
+//     subtiles (three at 8 bits). 64 rows of x do not fit LDS beside the ring, so x comes in
+//     chunks of 256 codes, double-buffered, and the accumulators of up to four
+//     128-row groups stay in registers over the chunks: a whole-tile block
+//     reads x and the weights once. Arithmetic and its order per output are
+//     those of the 16-slot form. 1999 tokens, 512 experts top 10, 2048 -> 512,
+//     4-bit: gate/up 356 -> 232 us (397 TFLOP/s);
+//     the fold's eight fmas per two MFMAs and the unpacking bound it now.
+
+// 16-slot subtiles of a wide tile: four (128 accumulator registers of the 256
+// a thread has); three with 8-bit codes, whose operands take more (four spill)
+constexpr int wide_subtiles(int bits) { return bits == 8 ? 3 : 4; }
+constexpr int kMWideK = 256;    // x codes of a chunk
+constexpr int kMWideRg = kMDownK / 128;  // 128-row groups at most
+
+template <int BITS, bool FP16>
+struct WideLds {
+  static constexpr int W = wide_subtiles(BITS);
+  alignas(16) uint16_t sx[2][W * kMTok * kMWideK];
+  alignas(16) uint8_t swt[2][8][RingSlot<BITS>::BYTES];
+  alignas(16) float sxs[kMWideK / 64][W * kMTok];
+  int tok[W * kMTok];
+};
+
+// one block's tile of NS subtiles
+template <int BITS, bool FP16, int NS>
+__device__ __forceinline__ void moe_gateup_wide_tile(const MoeArgs &a, const MoeMWs &w, WideLds<BITS, FP16> &L, int e,
+                                                     int row0, int cnt, int rg0, int nrg) {
+  constexpr int WAVES = 8, RPB = 16 * WAVES;
+  using R = RingSlot<BITS>;
+  using S = MfmaStep<BITS>;
+  constexpr int GU = R::GU, BPC = kMWideK / (64 * GU);  // batches of a chunk and row group
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r16 = lane & 15, g = lane >> 4;
+  const bool shared = e < 0;
+  const int rows = shared ? a.sinter : a.inter;
+  const DevBank &gbk = shared ? a.sgate : a.gate;
+  const DevBank &ubk = shared ? a.sup : a.up;
+  const size_t eo = shared ? 0 : (size_t)e;
+  const int nch = a.D / kMWideK;
+  const int jw0 = rg0 * RPB + wave * 16, rmax = rows - 1;
+  // copy sources as in the 16-slot form
+  const int lr = lane >> 3, sc = 16 * ((lane & 7) ^ lr);
+  const uint8_t *const gb = gbk.m.w + eo * gbk.w_stride + sc;
+  const uint8_t *const ub = ubk.m.w + eo * ubk.w_stride + sc;
+  const size_t grb = gbk.m.row_bytes, urb = ubk.m.row_bytes;
+  const uint16_t *ab0, *ab1;
+  int arl, ang0, ang1;
+  if constexpr (BITS == 4) {
+    ab0 = (lane < 32 ? gbk.m.sc : gbk.m.bi) + eo * gbk.p_stride + 2 * (lane & 1);
+    ab1 = (lane < 32 ? ubk.m.sc : ubk.m.bi) + eo * ubk.p_stride + 2 * (lane & 1);
+    arl = (lane & 31) >> 1;
+    ang0 = gbk.m.ng;
+    ang1 = ubk.m.ng;
+  } else {
+    const bool up = lane >= 32;
+    const bool bias = (lane >> 4) & 1;
+    ab0 = up ? (bias ? ubk.m.bi : ubk.m.sc) + eo * ubk.p_stride : (bias ? gbk.m.bi : gbk.m.sc) + eo * gbk.p_stride;
+    ab1 = ab0;
+    arl = lane & 15;
+    ang0 = up ? ubk.m.ng : gbk.m.ng;
+    ang1 = ang0;
+  }
+  const uint16_t *const xsrc = BITS == 4 ? w.xop : a.x;
+  const int hmax = a.inter > a.sinter ? a.inter : a.sinter, D = a.D;
+  const int nslots = a.B * a.k;
+  UnpackConsts kc;
+  kc.init();
+  const bf16x8_t ones = mfma_ones();
+  f32x4_t acc[kMWideRg][2][NS];
+#pragma unroll
+  for (int rg = 0; rg < kMWideRg; ++rg)
+#pragma unroll
+    for (int m = 0; m < 2; ++m)
+#pragma unroll
+      for (int t = 0; t < NS; ++t) acc[rg][m][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+  // rows past the tile repeat its last token and feed only unstored outputs
+  if (tid < NS * kMTok) L.tok[tid] = shared ? row0 - nslots + min(tid, cnt - 1) : w.tok[row0 + min(tid, cnt - 1)];
+  __syncthreads();
+  // the thread's granule of each subtile (32 a row; physical granule P of row
+  // m holds logical granule P ^ m)
+  const uint16_t *xr[NS];
+#pragma unroll
+  for (int t = 0; t < NS; ++t) {
+    const int m = tid >> 5, q = swz(m, tid & 31);
+    xr[t] = xsrc + (size_t)L.tok[16 * t + m] * D + 8 * q;
+  }
+  const uint32_t x0 = __builtin_amdgcn_readfirstlane(lds_addr(&L.sx[0][0]) + 1024u * wave);
+  constexpr uint32_t kXBuf = sizeof(L.sx[0]);
+  auto issue_x = [&](int c) {
+    const uint32_t d = __builtin_amdgcn_readfirstlane(x0 + (uint32_t)(c & 1) * kXBuf);
+#pragma unroll
+    for (int t = 0; t < NS; ++t) lds_copy16(xr[t] + (size_t)c * kMWideK, d + 8192u * t);
+  };
+  // the next batch to copy: chunk, row group, batch in both. Past the last
+  // one the copy repeats it into the other slot, which nothing reads then
+  const uint32_t ring0 = __builtin_amdgcn_readfirstlane(lds_addr(&L.swt[0][wave][0]));
+  int is = 0, ic = 0, ir = 0, ibl = 0;
+  auto issue_next = [&]() {
+    const uint32_t d = __builtin_amdgcn_readfirstlane(ring0 + (uint32_t)is * (WAVES * R::BYTES));
+    const int jr = jw0 + ir * RPB;
+    const int jl0 = min(jr + lr, rmax), jl1 = min(jr + 8 + lr, rmax), ja = min(jr + arl, rmax);
+    const int kb = ic * BPC + ibl;
+    const size_t o = (size_t)128 * kb;
+    const uint8_t *wr[4] = {gb + (size_t)jl0 * grb + o, gb + (size_t)jl1 * grb + o, ub + (size_t)jl0 * urb + o,
+                            ub + (size_t)jl1 * urb + o};
+    R::issue(d, wr, ab0 + (size_t)ja * ang0 + kb * GU, ab1 + (size_t)ja * ang1 + kb * GU);
+    is ^= 1;
+    if (++ibl == BPC) {
+      ibl = 0;
+      if (++ir == nrg) {
+        ir = 0;
+        if (++ic == nch) {  // stay on the last batch
+          ic = nch - 1;
+          ir = nrg - 1;
+          ibl = BPC - 1;
+        }
+      }
+    }
+  };
+  issue_x(0);
+  issue_next();
+  lds_dma_wait_behind<R::NI>();
+  __syncthreads();
+  int cs = 0;
+  for (int c = 0; c < nch; ++c) {
+    const uint16_t *sx = L.sx[c & 1];
+    // sums of x over the chunk's steps, one (step, subtile) pair per wave at a time
+    for (int v = wave; v < (kMWideK / 64) * NS; v += WAVES) {
+      const int u = v & 3, t = v >> 2;
+      bf16x8_t a0, a1;
+      S::a_ops(sx + (16 * t + r16) * kMWideK, (u * 64 + 16 * g) >> 3, r16, a0, a1);
+      const f32x4_t z = {0.f, 0.f, 0.f, 0.f};
+      f32x4_t xs = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, ones, z, 0, 0, 0);
+      xs = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, ones, xs, 0, 0, 0);
+      if (r16 == 0) *reinterpret_cast<float4 *>(&L.sxs[u][16 * t + 4 * g]) = make_float4(xs[0], xs[1], xs[2], xs[3]);
+    }
+    __syncthreads();
+    const bool more = c + 1 < nch;
+#pragma unroll
+    for (int rg = 0; rg < kMWideRg; ++rg) {
+      if (rg < nrg) {
+#pragma unroll
+        for (int bl = 0; bl < BPC; ++bl) {
+          issue_next();
+          // this batch has landed: behind it is the next batch, and at the
+          // chunk's second batch the next chunk's x as well
+          if (rg * BPC + bl == 1 && more) lds_dma_wait_behind<R::NI + NS>();
+          else lds_dma_wait_behind<R::NI>();
+          if (rg * BPC + bl == 0 && more) issue_x(c + 1);
+          const uint8_t *slot = &L.swt[cs][wave][0];
+          cs ^= 1;
+          uint32_t sw[2][GU / 2], bw[2][GU / 2];
+          R::aux(slot, r16, sw, bw);
+#pragma unroll
+          for (int u = 0; u < GU; ++u) {
+            const int ku = bl * GU + u;
+            bf16x8_t b0[2], b1[2];
+#pragma unroll
+            for (int m = 0; m < 2; ++m) {
+              SkRaw<BITS> rw;
+              R::raw(slot, m, u, r16, g, rw);
+              S::b_ops(rw, kc, b0[m], b1[m]);
+            }
+#pragma unroll
+            for (int t = 0; t < NS; ++t) {
+              bf16x8_t a0, a1;
+              S::a_ops(sx + (16 * t + r16) * kMWideK, (ku * 64 + 16 * g) >> 3, r16, a0, a1);
+              const f32x4_t z = {0.f, 0.f, 0.f, 0.f};
+              const float4 xv = *reinterpret_cast<const float4 *>(&L.sxs[ku][16 * t + 4 * g]);
+              const f32x4_t xs = {xv.x, xv.y, xv.z, xv.w};
+#pragma unroll
+              for (int m = 0; m < 2; ++m) {
+                f32x4_t d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b0[m], z, 0, 0, 0);
+                d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, b1[m], d, 0, 0, 0);
+                S::fold(acc[rg][m][t], d, xs, R::template word<FP16>(sw[m], u), R::template word<FP16>(bw[m], u));
+              }
+            }
+          }
+        }
+      }
+    }
+    // the next chunk's x is in LDS, and every wave is done with this one
+    if (nrg * BPC == 1) lds_dma_wait();
+    else lds_dma_wait_behind<R::NI>();
+    __syncthreads();
+  }
+  lds_dma_wait();  // no copy into LDS outlives the block
+#pragma unroll
+  for (int rg = 0; rg < kMWideRg; ++rg) {
+    const int jj = jw0 + rg * RPB + r16;
+    if (rg < nrg && jj < rows) {
+#pragma unroll
+      for (int t = 0; t < NS; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int m = 16 * t + 4 * g + i;
+          if (m < cnt) {
+            const float h = silu(acc[rg][0][t][i]) * acc[rg][1][t][i];
+            const uint32_t hi = f32_to_bf16_rne(h);
+            const uint32_t lo = f32_to_bf16_rne(h - bf16_to_f32(hi));
+            const size_t o = (size_t)(row0 + m) * hmax + S::op_pos(jj);
+            w.h_hi[o] = (uint16_t)hi;
+            w.h_lo[o] = (uint16_t)lo;
+          }
+        }
+    }
+  }
+}
+
+template <int BITS, bool FP16>
+__global__ __launch_bounds__(512, 1) void moe_gateup_wide_kernel(MoeArgs a, MoeMWs w, int ipt) {
+  __shared__ WideLds<BITS, FP16> L;
+  // whole-tile blocks first, one-group blocks for the last units (as above)
+  const int nt = __builtin_amdgcn_readfirstlane(*w.n_tiles);
+  const int units = nt * ipt;
+  const int nbt = units > kMGuSmallUnits ? (units - kMGuSmallUnits) / ipt : 0;
+  const int bid = blockIdx.x;
+  int tile = bid, rg0 = 0, nrg = ipt;
+  if (bid >= nbt) {
+    tile = nbt + (bid - nbt) / ipt;
+    rg0 = (bid - nbt) % ipt;
+    nrg = 1;
+  }
+  if (tile >= nt) return;
+  const int4 tr = w.tiles[tile];
+  const int e = __builtin_amdgcn_readfirstlane(tr.x);
+  const int row0 = __builtin_amdgcn_readfirstlane(tr.y);
+  const int cnt = __builtin_amdgcn_readfirstlane(tr.z);
+  const int rows = e < 0 ? a.sinter : a.inter;
+  if (rg0 * 128 >= rows) return;
+  nrg = min(nrg, (rows + 127) / 128 - rg0);
+  switch ((cnt + kMTok - 1) / kMTok) {
+    case 1: moe_gateup_wide_tile<BITS, FP16, 1>(a, w, L, e, row0, cnt, rg0, nrg); break;
+    case 2: moe_gateup_wide_tile<BITS, FP16, 2>(a, w, L, e, row0, cnt, rg0, nrg); break;
+    case 3: moe_gateup_wide_tile<BITS, FP16, 3>(a, w, L, e, row0, cnt, rg0, nrg); break;
+    default:
+      if constexpr (wide_subtiles(BITS) == 4) moe_gateup_wide_tile<BITS, FP16, 4>(a, w, L, e, row0, cnt, rg0, nrg);
+  }
+}
+
+// ---------------------------------------------------------------------------
 // 4. down: block = (tile, 128 rows), wave = 2 x 16 rows, K <= 512: h copied
 //    into LDS first, then every scale/bias and weight load of the wave, and
 //    each step waits only for its own weights
@@ -939,19 +1190,25 @@ __global__ __launch_bounds__(256) void moe_down_mfma_kernel(MoeArgs a, MoeMWs w,
 //     CUs whose whole-tile blocks end first take the small ones (config-5
 //     chunk: 118-119 us per layer with 512-row blocks only, 98 us so; 110 us
 //     with 128 small units, 103 with 512).
+//
+//     MT = 2 (wide tiles, in parts of 32 slots; a two-slot ring): h of 32 rows,
+//     the codes unpacked once for both 16-slot halves. A pair's stores count
+//     in vmcnt behind the copies; waiting for the copies alone made each pair
+//     wait for its own stores too (512-token block 263 -> 258 us, 160 tokens
+//     250 -> 239).
 
 constexpr int kMDownLdsRows = 512;      // rows of a small block (32 x 2 pairs x 8 waves)
 constexpr int kMDownSmallUnits = 256;   // 512-row units left to small blocks (one round on 256 CUs)
 
-template <int BITS, bool FP16>
+template <int BITS, bool FP16, int MT>
 __global__ __launch_bounds__(512, 1) void moe_down_lds_kernel(MoeArgs a, MoeMWs w, int upt) {
   constexpr int WAVES = 8, NT = WAVES * 64;
   using R = RingSlot<BITS>;
-  constexpr int GU = R::GU, NB = 3;
+  constexpr int GU = R::GU, NB = MT == 1 ? 3 : 2;
   constexpr int NS = kMDownK / 64;      // steps at most
   constexpr int KBM = NS / GU;           // batches per pair at most
-  __shared__ __align__(16) uint16_t shi[kMTok * kMDownK];
-  __shared__ __align__(16) uint16_t slo[kMTok * kMDownK];
+  __shared__ __align__(16) uint16_t shi[MT * kMTok * kMDownK];
+  __shared__ __align__(16) uint16_t slo[MT * kMTok * kMDownK];
   __shared__ __align__(16) uint8_t swt[NB][WAVES][R::BYTES];
   using S = MfmaStep<BITS>;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -959,7 +1216,8 @@ __global__ __launch_bounds__(512, 1) void moe_down_lds_kernel(MoeArgs a, MoeMWs 
   const int r16 = lane & 15, g = lane >> 4;
   // blocks [0, nbt) take whole tiles; then the tiles from nbt on in 512-row
   // units (upt = ceil(D / 512) per tile; the grid holds max_tiles x upt)
-  const int nt = __builtin_amdgcn_readfirstlane(*w.n_tiles);
+  constexpr int PPT = MT == 1 ? 1 : (wide_subtiles(BITS) + MT - 1) / MT;  // parts per tile
+  const int nt = PPT * __builtin_amdgcn_readfirstlane(*w.n_tiles);
   const int units = nt * upt;
   const int nbt = units > kMDownSmallUnits ? (units - kMDownSmallUnits) / upt : 0;
   const int bid = blockIdx.x;
@@ -974,10 +1232,12 @@ __global__ __launch_bounds__(512, 1) void moe_down_lds_kernel(MoeArgs a, MoeMWs 
     npw = 2;
   }
   if (tile >= nt) return;
-  const int4 tr = w.tiles[tile];
+  const int4 tr = w.tiles[tile / PPT];
+  const int part = MT * kMTok * (tile % PPT);
   const int e = __builtin_amdgcn_readfirstlane(tr.x);
-  const int row0 = __builtin_amdgcn_readfirstlane(tr.y);
-  const int cnt = __builtin_amdgcn_readfirstlane(tr.z);
+  const int row0 = __builtin_amdgcn_readfirstlane(tr.y) + part;
+  const int cnt = min(__builtin_amdgcn_readfirstlane(tr.z) - part, MT * kMTok);
+  if (cnt <= 0) return;  // the tile ends before this part
   const bool shared = e < 0;
   const DevBank &dbk = shared ? a.sdown : a.down;
   const int K = shared ? a.sinter : a.inter;
@@ -1042,7 +1302,7 @@ __global__ __launch_bounds__(512, 1) void moe_down_lds_kernel(MoeArgs a, MoeMWs 
   {
     // stage h (hi, lo) of the tile's rows (physical granule P of row m holds
     // logical granule P ^ (m & 15))
-    constexpr int NQ = kMTok * kMDownK / 8 / NT;
+    constexpr int NQ = MT * kMTok * kMDownK / 8 / NT;
     const int gpr = K >> 3;
     auto dma = [&](int base) {
       const int pg = base + lane;
@@ -1058,38 +1318,49 @@ __global__ __launch_bounds__(512, 1) void moe_down_lds_kernel(MoeArgs a, MoeMWs 
   }
   // the ring's first two batches behind the h copies (a wave with no rows
   // inside D copies clamped rows and stores nothing)
-  issue_next();
-  issue_next();
-  lds_dma_wait_behind<2 * R::NI>();
+#pragma unroll
+  for (int i = 0; i < NB - 1; ++i) issue_next();
+  lds_dma_wait_behind<(NB - 1) * R::NI>();
   __syncthreads();
   UnpackConsts kc;
   kc.init();
   const bf16x8_t ones = mfma_ones();
   // sum of h over each step's 64 k (hi and lo): the fold's bias term
-  f32x4_t xs[NS];
+  f32x4_t xs[MT][NS];
 #pragma unroll
-  for (int u = 0; u < NS; ++u) {
-    if (u < kbn * GU) {
-      bf16x8_t h0, h1, l0, l1;
-      const int q0 = (u * 64 + 16 * g) >> 3;
-      S::a_ops(shi + r16 * K, q0, r16, h0, h1);
-      S::a_ops(slo + r16 * K, q0, r16, l0, l1);
-      const f32x4_t z = {0.f, 0.f, 0.f, 0.f};
-      xs[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(h0, ones, z, 0, 0, 0);
-      xs[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(h1, ones, xs[u], 0, 0, 0);
-      xs[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(l0, ones, xs[u], 0, 0, 0);
-      xs[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(l1, ones, xs[u], 0, 0, 0);
+  for (int t = 0; t < MT; ++t)
+#pragma unroll
+    for (int u = 0; u < NS; ++u) {
+      if (u < kbn * GU) {
+        bf16x8_t h0, h1, l0, l1;
+        const int q0 = (u * 64 + 16 * g) >> 3;
+        S::a_ops(shi + (16 * t + r16) * K, q0, r16, h0, h1);
+        S::a_ops(slo + (16 * t + r16) * K, q0, r16, l0, l1);
+        f32x4_t v = {0.f, 0.f, 0.f, 0.f};
+        v = __builtin_amdgcn_mfma_f32_16x16x32_bf16(h0, ones, v, 0, 0, 0);
+        v = __builtin_amdgcn_mfma_f32_16x16x32_bf16(h1, ones, v, 0, 0, 0);
+        v = __builtin_amdgcn_mfma_f32_16x16x32_bf16(l0, ones, v, 0, 0, 0);
+        xs[t][u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(l1, ones, v, 0, 0, 0);
+      }
     }
-  }
+  constexpr int kStores = 8 * MT;  // stores of a pair
+  auto yr = __builtin_amdgcn_make_buffer_rsrc(w.y + (size_t)row0 * a.D, 0, 4 * cnt * a.D, 0x00027000);
   int cs = 0;  // ring slot of the batch multiplied
   for (int p = 0; p < npw; ++p) {
-    f32x4_t acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+    f32x4_t acc[2][MT];
+#pragma unroll
+    for (int m = 0; m < 2; ++m)
+#pragma unroll
+      for (int t = 0; t < MT; ++t) acc[m][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int kb = 0; kb < KBM; ++kb) {
       if (kb < kbn) {
         // two batches in flight behind this one
         issue_next();
-        lds_dma_wait_behind<2 * R::NI>();
+        // behind this batch: the copies of the next ones and, in the NB - 1
+        // batches after a pair's stores, those stores
+        if (p > 0 && kb < NB - 1) lds_dma_wait_behind<(NB - 1) * R::NI + kStores>();
+        else lds_dma_wait_behind<(NB - 1) * R::NI>();
         const uint8_t *slot = &swt[cs][wave][0];
         cs = cs == NB - 1 ? 0 : cs + 1;
         uint32_t sw[2][GU / 2], bw[2][GU / 2];
@@ -1098,35 +1369,41 @@ __global__ __launch_bounds__(512, 1) void moe_down_lds_kernel(MoeArgs a, MoeMWs 
         for (int ul = 0; ul < GU; ++ul) {
           const int u = kb * GU + ul;
           const int q0 = (u * 64 + 16 * g) >> 3;
-          bf16x8_t h0, h1, l0, l1;
-          S::a_ops(shi + r16 * K, q0, r16, h0, h1);
-          S::a_ops(slo + r16 * K, q0, r16, l0, l1);
-          const f32x4_t z = {0.f, 0.f, 0.f, 0.f};
+          bf16x8_t b0[2], b1[2];
 #pragma unroll
           for (int m = 0; m < 2; ++m) {
             SkRaw<BITS> rw;
-            bf16x8_t b0, b1;
             R::raw(slot, m, ul, r16, g, rw);
-            S::b_ops(rw, kc, b0, b1);
-            f32x4_t d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(h0, b0, z, 0, 0, 0);
-            d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(h1, b1, d, 0, 0, 0);
-            d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(l0, b0, d, 0, 0, 0);
-            d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(l1, b1, d, 0, 0, 0);
-            S::fold(acc[m], d, xs[u], R::template word<FP16>(sw[m], ul),
-                    R::template word<FP16>(bw[m], ul));
+            S::b_ops(rw, kc, b0[m], b1[m]);
+          }
+#pragma unroll
+          for (int t = 0; t < MT; ++t) {
+            bf16x8_t h0, h1, l0, l1;
+            S::a_ops(shi + (16 * t + r16) * K, q0, r16, h0, h1);
+            S::a_ops(slo + (16 * t + r16) * K, q0, r16, l0, l1);
+            const f32x4_t z = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int m = 0; m < 2; ++m) {
+              f32x4_t d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(h0, b0[m], z, 0, 0, 0);
+              d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(h1, b1[m], d, 0, 0, 0);
+              d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(l0, b0[m], d, 0, 0, 0);
+              d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(l1, b1[m], d, 0, 0, 0);
+              S::fold(acc[m][t], d, xs[t][u], R::template word<FP16>(sw[m], ul), R::template word<FP16>(bw[m], ul));
+            }
           }
         }
       }
     }
+    // the pair's outputs; the resource drops rows from cnt on, so that every
+    // wave issues exactly kStores stores (the waits above count them)
 #pragma unroll
     for (int m = 0; m < 2; ++m) {
       const int d = jw + 32 * p + 16 * m + r16;
-      if (d < a.D) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int t = 4 * g + i;
-          if (t < cnt) w.y[(size_t)(row0 + t) * a.D + d] = acc[m][i];
-        }
+      for (int i = 0; i < 4 * MT; ++i) {
+        const int t = 16 * (i >> 2) + 4 * g + (i & 3);
+        const int o = d < a.D && t < cnt ? 4 * (t * a.D + d) : -4;
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[m][i >> 2][i & 3]), yr, o, 0, 0);
       }
     }
   }
@@ -1244,6 +1521,38 @@ bool moe_mfma_supported(const MoeArgs &a) {
   return true;
 }
 
+// tiles of `ts` slots at most: every routed expert and the shared one may end
+// in a part of a tile
+static int tiles_bound(const MoeArgs &a, int ts) {
+  const int nsl = a.B * a.k;
+  return nsl / ts + (nsl < a.E ? nsl : a.E) + (a.B + ts - 1) / ts;
+}
+
+// Whether tiles hold up to 64 (8-bit: 48) slots: both passes on the LDS
+// kernels (4/8-bit, groups of 64, whole batches of the down K), and
+//  * 32 slots an expert, that is more than two 16-slot tiles (whole block in us,
+//    16-slot -> wide tiles, 512 experts top 10, popularity rank^-1.1: 4-bit 27
+//    an expert 458 -> 472, 39: 587 -> 548; uniform 457 -> 393, 605 -> 482;
+//    8-bit 27: 634 -> 610, 39: 803 -> 703; uniform 666 -> 522, 877 -> 633);
+//  * enough (slot, 128-row group) pairs for the 256 CUs, a wide block being
+//    several times as long: 96 each, 60 with 8-bit codes, where the 16-slot
+//    form moves twice the bytes (512 rows: 64 experts top 6, 4-bit 3000 slots
+//    75 -> 98, 5400: 109 -> 108, 8400: 149 -> 117, 8-bit 3000 slots 87 -> 95,
+//    5400: 129 -> 108; 128 experts top 8 skewed, 4000 slots 4-bit 172 -> 186,
+//    8-bit 236 -> 210).
+static bool wide_tiles(const MoeArgs &a) {
+  const int bits = a.gate.m.bits;
+  if (a.B <= kMGuSmallB || (bits != 4 && bits != 8)) return false;
+  const bool sh = a.sgate.m.w != nullptr;
+  if (a.gate.m.gs != 64 || a.up.m.gs != 64 || a.down.m.gs != 64 ||
+      (sh && (a.sgate.m.gs != 64 || a.sup.m.gs != 64 || a.sdown.m.gs != 64)))
+    return false;
+  const int kb = 128 * 8 / bits;
+  if (a.inter % kb != 0 || (sh && a.sinter % kb != 0) || a.D % kMWideK != 0) return false;
+  const long long slots = (long long)a.B * a.k;
+  return slots >= 32LL * a.E && slots * (a.inter / 128) >= 256LL * (bits == 8 ? 60 : 96);
+}
+
 template <int BITS, int WV>
 static hipError_t moe_gateup_launch(const MoeArgs &a, const MoeMWs &w, hipStream_t st) {
   const int kmax = a.inter > a.sinter ? a.inter : a.sinter;
@@ -1255,6 +1564,12 @@ static hipError_t moe_gateup_launch(const MoeArgs &a, const MoeMWs &w, hipStream
     const dim3 grid(w.max_tiles * ipt), block(WV * 64);
     if constexpr (WV == 8 && (BITS == 4 || BITS == 8)) {
       // the large-batch shape with the weights staged in LDS (groups of 64)
+      if (wide_tiles(a)) {
+        const dim3 wgrid(tiles_bound(a, wide_subtiles(BITS) * kMTok) * ipt);
+        if (a.gate.m.fp16) hipLaunchKernelGGL((moe_gateup_wide_kernel<BITS, true>), wgrid, block, 0, st, a, w, ipt);
+        else hipLaunchKernelGGL((moe_gateup_wide_kernel<BITS, false>), wgrid, block, 0, st, a, w, ipt);
+        return hipGetLastError();
+      }
       if (gs64 && a.gate.m.gs == 64) {
         if (a.gate.m.fp16) hipLaunchKernelGGL((moe_gateup_lds_kernel<BITS, true>), grid, block, 0, st, a, w, ipt);
         else hipLaunchKernelGGL((moe_gateup_lds_kernel<BITS, false>), grid, block, 0, st, a, w, ipt);
@@ -1282,10 +1597,16 @@ static hipError_t moe_down_launch(const MoeArgs &a, const MoeMWs &w, hipStream_t
                      (!a.sdown.m.w || (a.sdown.m.gs == 64 && a.sinter % KB == 0));
     if (lds) {
       const int upt = (a.D + kMDownLdsRows - 1) / kMDownLdsRows;
+      if (wide_tiles(a)) {
+        const dim3 wgrid(tiles_bound(a, wide_subtiles(BITS) * kMTok) * ((wide_subtiles(BITS) + 1) / 2) * upt);
+        if (a.down.m.fp16) hipLaunchKernelGGL((moe_down_lds_kernel<BITS, true, 2>), wgrid, dim3(512), 0, st, a, w, upt);
+        else hipLaunchKernelGGL((moe_down_lds_kernel<BITS, false, 2>), wgrid, dim3(512), 0, st, a, w, upt);
+        return hipGetLastError();
+      }
       if (a.down.m.fp16)
-        hipLaunchKernelGGL((moe_down_lds_kernel<BITS, true>), dim3(w.max_tiles * upt), dim3(512), 0, st, a, w, upt);
+        hipLaunchKernelGGL((moe_down_lds_kernel<BITS, true, 1>), dim3(w.max_tiles * upt), dim3(512), 0, st, a, w, upt);
       else
-        hipLaunchKernelGGL((moe_down_lds_kernel<BITS, false>), dim3(w.max_tiles * upt), dim3(512), 0, st, a, w, upt);
+        hipLaunchKernelGGL((moe_down_lds_kernel<BITS, false, 1>), dim3(w.max_tiles * upt), dim3(512), 0, st, a, w, upt);
       return hipGetLastError();
     }
   }
@@ -1328,7 +1649,7 @@ int launch_moe_mfma(const MoeArgs &a, hipStream_t st) {
     else hipLaunchKernelGGL((moe_mroute_kernel<16, false>), rgrid, dim3(256), 0, st, a, w);
   }
   if (hipGetLastError() != hipSuccess) return -1;
-  hipLaunchKernelGGL(moe_mgroup_kernel, dim3(1), dim3(kMGroupThreads), 0, st, a, w);
+  hipLaunchKernelGGL(moe_mgroup_kernel, dim3(1), dim3(kMGroupThreads), 0, st, a, w, wide_tiles(a) ? wide_subtiles(a.gate.m.bits) * kMTok : kMTok);
   if (hipGetLastError() != hipSuccess) return -1;
   switch (a.gate.m.bits) {
     case 4: return moe_mfma_launch_bits<4>(a, w, st);

@@ -19,7 +19,7 @@ HOT = {
     "moe.hip": [r"moe_gateup_kernelILi4ELi1E", r"moe_down_kernelILi4ELi16E", r"moe_route_tok_kernel",
                 r"moe_group_kernel", r"moe_combine_kernel"],
     "moe_fused.hip": [r"moe_fused_b1_kernelILi4ELi1ELi16E"],
-    "moe_mfma.hip": [r"moe_gateup_lds_kernel", r"moe_down_lds_kernel", r"moe_gateup_mfma_kernelILi4E",
+    "moe_mfma.hip": [r"moe_gateup_lds_kernel", r"moe_gateup_wide_kernel", r"moe_down_lds_kernel", r"moe_gateup_mfma_kernelILi4E",
                      r"moe_down_mfma_kernelILi4E", r"moe_mroute_kernel", r"moe_mgroup_kernel",
                      r"moe_mcombine_kernel"],
 }

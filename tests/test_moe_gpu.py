@@ -505,6 +505,39 @@ def test_moe_prefill_whole_tile_blocks(gpu, bits, fp16, D, sinter):
         assert normwise_rel(out32[t], out_d[t]) <= 5e-5
 
 
+@pytest.mark.parametrize("bits,fp16,E,k,B,D,inter,sinter", [
+    (4, False, 64, 8, 801, 2048, 512, 256), (4, True, 32, 16, 799, 768, 256, 512),
+    (8, False, 64, 8, 701, 1024, 384, 512), (8, True, 16, 8, 1999, 256, 128, 128),
+    (4, False, 48, 8, 801, 4096, 512, 0)])
+def test_moe_prefill_wide_tiles(gpu, bits, fp16, E, k, B, D, inter, sinter):
+    """Experts with more than 32 slots on average take tiles of 64 (8-bit: 48)
+    slots: skewed routes, so that tiles of every number of subtiles and
+    remainder occur; one to sixteen x chunks, one to four row groups, one
+    batch per chunk and several; no shared expert. A sample against the
+    oracle, every token against the per-token path."""
+    import torch
+    from logan_amd import _lib
+
+    print(f"moe wide tiles bits={bits} fp16={fp16} E={E} B={B} D={D} inter={inter}", flush=True)
+    layer = Layer(torch, E, k, D, inter, bits, 64, seed=131 + bits + D, fp16=fp16, shared=sinter > 0,
+                  sinter=sinter or None)
+    rng = np.random.default_rng(132 + D)
+    xb = make_x(rng, B, D)
+    lb = make_logits(rng, B, E, zipf_s=1.1)
+    out32, idx, w = run_layer(torch, layer, xb, lb, torch.float32)
+    out32 = out32.cpu().numpy()
+    _check_tokens(layer, xb, lb, out32, idx, w, range(0, B, 53))
+    _lib.lib().logan_hip_set_moe_mfma_min_batch(1 << 20)
+    try:
+        out_d, idx_d, _ = run_layer(torch, layer, xb, lb, torch.float32)
+    finally:
+        _lib.lib().logan_hip_set_moe_mfma_min_batch(0)
+    np.testing.assert_array_equal(idx, idx_d)
+    out_d = out_d.cpu().numpy()
+    for t in range(B):
+        assert normwise_rel(out32[t], out_d[t]) <= 5e-5
+
+
 @pytest.mark.parametrize("mfma_min_b", [1 << 20], indirect=True)
 def test_moe_large_batch_per_token_passes(gpu, mfma_min_b):
     """With the MFMA path off, B = 100 runs the per-token path in passes of
