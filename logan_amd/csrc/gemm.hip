@@ -303,6 +303,15 @@ __device__ __forceinline__ void q_wait() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
+// wait until all but the last N LDS operations of this wave are done (they
+// return in order). A copy into LDS is unseen by the compiler, which places no
+// wait between the reads of a stage and the copies that overwrite it.
+template <int N>
+__device__ __forceinline__ void q_wait_lds() {
+  static_assert(N >= 0 && N <= 15, "lgkmcnt is 4 bits");
+  asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(N) : "memory");
+}
+
 // Geometry of one instantiation.
 template <int BITS, int MI, bool GS64>
 struct QTile {
@@ -583,7 +592,8 @@ __global__ __launch_bounds__(512, 2) void affine_qmm_tile_kernel(QmmMulti p, int
     }
   };
   // Pipeline. Step t's iteration waits for its own copies of step t + 1 (those
-  // of the NST - 3 steps after it may be in flight), meets the barrier (step
+  // of the NST - 3 steps after it may be in flight) and for its LDS reads but
+  // the MI of the next x operands, meets the barrier (step
   // t + 1 is then readable, and nobody reads x of step t - 1 or codes of step t
   // any more) and, between its MFMAs, issues the copies of step t + NST - 1; a
   // chunk's first step also copies the next chunk's scale / bias words. While
@@ -606,6 +616,7 @@ __global__ __launch_bounds__(512, 2) void affine_qmm_tile_kernel(QmmMulti p, int
   bf16x8 xa[MI];
   uint32_t wf[2][4];
   read_raw(0, raw);
+  __builtin_amdgcn_sched_barrier(0);  // ahead of x's reads: the wait below counts those alone
 #pragma unroll
   for (int i = 0; i < MI; ++i) xa[i] = *reinterpret_cast<const bf16x8 *>(xrd[0] + 4096 * i);
   {
@@ -660,12 +671,14 @@ __global__ __launch_bounds__(512, 2) void affine_qmm_tile_kernel(QmmMulti p, int
     __builtin_amdgcn_sched_barrier(0);
     if ((unsigned)(cs - 1) < (unsigned)(NST - 3)) q_wait<(NST - 3) * G::L + G::NA>();
     else q_wait<(NST - 3) * G::L>();
+    q_wait_lds<MI>();
     __builtin_amdgcn_s_barrier();
     step(std::true_type{}, t);
   }
   for (; t < nst; ++t) {
     __builtin_amdgcn_sched_barrier(0);
     q_wait<0>();
+    q_wait_lds<MI>();
     __builtin_amdgcn_s_barrier();
     step(std::false_type{}, t);
   }
