@@ -899,6 +899,9 @@ __device__ __forceinline__ void moe_gateup_wide_tile(const MoeArgs &a, const Moe
   const uint32_t ring0 = __builtin_amdgcn_readfirstlane(lds_addr(&L.swt[0][wave][0]));
   int is = 0, ic = 0, ir = 0, ibl = 0;
   auto issue_next = [&]() {
+    // the slot's last reads are done (the compiler does not see the copy: with
+    // 8-bit codes it left the scale / bias reads in flight here)
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     const uint32_t d = __builtin_amdgcn_readfirstlane(ring0 + (uint32_t)is * (WAVES * R::BYTES));
     const int jr = jw0 + ir * RPB;
     const int jl0 = min(jr + lr, rmax), jl1 = min(jr + 8 + lr, rmax), ja = min(jr + arl, rmax);

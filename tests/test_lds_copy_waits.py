@@ -133,3 +133,17 @@ def test_qmm_tile_reads_complete_at_the_barriers(hipcc, tmp_path):
         if most > mi:
             bad[name] = most
     assert not bad
+
+
+def test_moe_ring_reads_complete_at_the_copies(hipcc, tmp_path):
+    """A wave's reads of its ring complete before it copies the next batch
+    into the slot it has read."""
+    ks = _kernels(CSRC / "moe_mfma.hip", "(lds|wide)_kernel", tmp_path)
+    assert ks
+    bad = {}
+    for name, lines in ks.items():
+        most, sites = reads_in_flight(lines, "global_load_lds")
+        assert sites, name
+        if most:
+            bad[name] = most
+    assert not bad
