@@ -1,10 +1,12 @@
-"""CPU check of the hot MoE kernels' private (scratch) memory, from the
+"""CPU check of the hot kernels' private (scratch) memory, from the
 compiler's resource report for gfx950.
 
 An index the compiler cannot resolve into the by-value MoeArgs kernel
 argument makes it copy the whole struct to scratch in every thread (the
 per-token kernels ran 4x slower that way); spills show up the same way.
-The kernels listed here must use no scratch at all.
+The kernels listed here must use no scratch at all; where waits count
+vector-memory instructions (the tile product, the LDS rings), a spill would
+also break the count.
 """
 import re
 import subprocess
@@ -16,6 +18,7 @@ from logan_amd import build
 
 CSRC = Path(build.CSRC)
 HOT = {
+    "gemm.hip": [r"affine_qmm_tile_kernelILi%dELi%dE" % (b, mi) for b in (4, 5, 6, 8) for mi in (1, 2, 4, 6, 8)],
     "moe.hip": [r"moe_gateup_kernelILi4ELi1E", r"moe_down_kernelILi4ELi16E", r"moe_route_tok_kernel",
                 r"moe_group_kernel", r"moe_combine_kernel"],
     "moe_fused.hip": [r"moe_fused_b1_kernelILi4ELi1ELi16E"],
