@@ -232,14 +232,22 @@ int logan_hip_affine_qmm(const LoganHipAffine *w, const void *x, int M, int x_st
 
 /* Up to 8 matrices that read the same x (q/k/v, qkvz/ba of a prefill
  * chunk) as one product: ys[i][M][O_i] = x . bf16(W_i)^T, each as
- * logan_hip_affine_qmm. With 16-byte aligned weights (5-bit: 4-byte) and
- * 4-byte aligned scales and biases their column tiles form one grid (the
- * reference encodes its batch of products into one command buffer,
- * backend_metal.mm:2290-2493); otherwise one launch per matrix. Every matrix has the same I, bits, group_size and aux type. 1
+ * logan_hip_affine_qmm. Their column tiles form one grid (the reference
+ * encodes its batch of products into one command buffer,
+ * backend_metal.mm:2290-2493); for M <= 64 only with 16-byte aligned weights
+ * (5-bit: 4-byte) and 4-byte aligned scales and biases, otherwise one launch
+ * per matrix. Every matrix has the same I, bits, group_size and aux type. 1
  * ok, 0 unsupported, -1 launch failure. Split grids share
  * logan_hip_affine_qmm's scratch slots and their cross-stream ordering. */
 int logan_hip_affine_qmm_multi(const LoganHipAffine *ws, int count, const void *x, int M,
                                int x_stride, void *const *ys, int y_dtype, void *stream);
+
+/* How a product of these operands runs, on the host alone: route[0] 0: the 64
+ * x 64 kernel, one launch per matrix (route[1], route[2] are 0); 1: one grid
+ * of the tile kernel; 2: of its form for operands off the alignment above;
+ * route[1] its rows per tile, route[2] its k ranges. 1 ok, 0 unsupported. */
+int logan_hip_affine_qmm_route(const LoganHipAffine *ws, int count, int M, int x_stride,
+                               int *route);
 
 /* SwiGLU between a dense gate/up pair and the down projection, in place:
  * g[i] = silu(g[i]) * u[i], silu(v) = v / (1 + exp(-v)), f32 arithmetic

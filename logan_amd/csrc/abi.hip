@@ -1290,6 +1290,19 @@ int logan_hip_affine_qmm_multi(const LoganHipAffine *ws, int count, const void *
                                              reinterpret_cast<hipStream_t>(stream)));
 }
 
+int logan_hip_affine_qmm_route(const LoganHipAffine *ws, int count, int M, int x_stride, int *route) {
+  if (!ws || !route || count <= 0 || count > 8 || M <= 0) return 0;
+  lh::DevMat ms[8];
+  for (int i = 0; i < count; ++i) {
+    if (!affine_ok(&ws[i]) || x_stride < ws[i].I) return 0;
+    ms[i] = devmat(ws[i]);
+  }
+  int r[3];
+  if (!lh::affine_qmm_route(ms, count, x_stride, M, r)) return 0;
+  for (int i = 0; i < 3; ++i) route[i] = r[i];
+  return 1;
+}
+
 int logan_hip_silu_mul(void *g, const void *u, long long n, int dtype, void *stream) {
   if (!g || !u || n <= 0) return 0;
   if (dtype != LOGAN_HIP_F32 && dtype != LOGAN_HIP_BF16) return 0;

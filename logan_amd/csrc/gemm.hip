@@ -4,9 +4,10 @@
 // dequantised weight rounded to bf16 in threadgroup memory, bf16 x bf16
 // products accumulated in f32, bf16 output).
 //
-// affine_qmm_tile_kernel serves every product whose rows allow 16-byte copies;
-// affine_qmm_kernel (64 x 64 tiles, 4 waves, dword loads) the rest (packed
-// rows off 16 bytes, scale / bias rows off 4) and the smallest products.
+// affine_qmm_tile_kernel serves all but the smallest products and, of those
+// whose operands are off the alignment of its wider copies (packed rows off 16
+// bytes, scales or biases off 4), the ones of up to 64 rows: those take
+// affine_qmm_kernel (64 x 64 tiles, 4 waves, dword loads).
 // Operand layout of v_mfma_f32_32x32x16_bf16 (checked on the device): lane l
 // holds row (col) l % 32 and 8 consecutive k at offset 8 * (l / 32) of each
 // 16-wide k slice; the result's element i of lane l is row
@@ -312,8 +313,10 @@ __device__ __forceinline__ void q_wait_lds() {
   asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(N) : "memory");
 }
 
-// Geometry of one instantiation.
-template <int BITS, int MI, bool GS64>
+// Geometry of one instantiation. ALN: packed rows start on 16 bytes (5 bits: on
+// 4), scales and biases on 4. Without it the codes come by dwords and the
+// sidecars may start on the second half of one.
+template <int BITS, int MI, bool GS64, bool ALN>
 struct QTile {
   static constexpr int BM = 32 * MI;               // tile rows
   static constexpr int RB = 8 * BITS;              // code bytes per row and step
@@ -324,15 +327,16 @@ struct QTile {
   static constexpr int NWS = NST - 1;
   static constexpr int AUX0 = NST * XB + NWS * WB;
   // steps of a chunk of scale / bias words, dwords per row of it: CS groups of
-  // 64 that may start inside a dword; groups of 32 start on one
-  static constexpr int ndw(int cs) { return GS64 ? cs / 2 + 1 : cs; }
+  // 64 that may start inside a dword; groups of 32 start on one (when ALN)
+  static constexpr int ndw(int cs) { return GS64 ? cs / 2 + 1 : cs + !ALN; }
   static constexpr int ab(int cs) { return 2 * kTN * ndw(cs) * 4; }  // [scale, bias][128][ndw]
   static constexpr int CS = AUX0 + 2 * ab(8) <= 163840 ? 8 : AUX0 + 2 * ab(6) <= 163840 ? 6 : 4;
   static constexpr int NDW = ndw(CS);
   static constexpr int AB = ab(CS);
   static constexpr int XI = BM / 8;                // x copies (1 KB) of a stage
   static constexpr int LX = (XI + 7) / 8;          // per wave
-  static constexpr int WI = BITS == 5 ? 20 : BITS; // code copies (1 KB; 5-bit 256 bytes)
+  static constexpr bool W16 = ALN && BITS != 5;    // code copies of 1 KB, else of 256 bytes
+  static constexpr int WI = W16 ? BITS : 4 * BITS;
   static constexpr int LW = (WI + 7) / 8;
   static constexpr int L = LX + LW;
   static constexpr int NA = (4 * NDW + 7) / 8;     // scale / bias copies per wave and chunk
@@ -423,10 +427,11 @@ struct QRun {
 };
 
 // GS64: groups of 64 codes (a group per step); else any multiple of 32
-template <int BITS, int MI, bool GS64, bool FP16>
+// (FP16: of the aligned form; the other takes p.fp16)
+template <int BITS, int MI, bool GS64, bool FP16, bool ALN>
 __global__ __launch_bounds__(512, 2) void affine_qmm_tile_kernel(QmmMulti p, int mtiles, int ntiles,
                                                                  int ksteps, int slot) {
-  using G = QTile<BITS, MI, GS64>;
+  using G = QTile<BITS, MI, GS64, ALN>;
   constexpr int BM = G::BM, NST = G::NST, CS = G::CS, NDW = G::NDW;
   __shared__ __align__(256) uint8_t smem[G::BYTES];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -469,16 +474,17 @@ __global__ __launch_bounds__(512, 2) void affine_qmm_tile_kernel(QmmMulti p, int
   for (int i = 0; i < G::LW; ++i) {
     const int c = (wave * G::LW + i) % G::WI, u = 64 * c + lane;
     int r, b;
-    if constexpr (BITS == 5) {
-      r = u / 10;
-      b = 4 * (u % 10);
+    if constexpr (!G::W16) {
+      r = u / (G::RB / 4);
+      const int q = u % (G::RB / 4);
+      b = BITS == 8 ? 16 * ((q >> 2) ^ ((r >> 2) & 3)) + 4 * (q & 3) : 4 * q;
     } else {
       r = u / (G::RB / 16);
       const int q = u % (G::RB / 16);
       b = 16 * (BITS == 8 ? q ^ ((r >> 2) & 3) : q);
     }
     woff[i] = (uint32_t)(min(r, N - 1 - bn0) * (int)mat.row_bytes + b);
-    wdst[i] = lds0 + NST * G::XB + (BITS == 5 ? 256 : 1024) * c;
+    wdst[i] = lds0 + NST * G::XB + (G::W16 ? 1024 : 256) * c;
   }
   const uint8_t *xsrc = reinterpret_cast<const uint8_t *>(p.x + (size_t)bm0 * p.x_stride + kb);
   const uint8_t *wsrc = mat.w + (size_t)bn0 * mat.row_bytes + (size_t)kb * BITS / 8;
@@ -490,8 +496,8 @@ __global__ __launch_bounds__(512, 2) void affine_qmm_tile_kernel(QmmMulti p, int
       q_copy16(xsrc, xoff[i], xdst + xst + 1024 * i);
     } else {
       const int i = k < G::LX ? 0 : k - G::LX;
-      if constexpr (BITS == 5) q_copy4(wsrc, woff[i], wdst[i] + wst);
-      else q_copy16(wsrc, woff[i], wdst[i] + wst);
+      if constexpr (G::W16) q_copy16(wsrc, woff[i], wdst[i] + wst);
+      else q_copy4(wsrc, woff[i], wdst[i] + wst);
     }
   };
   auto next = [&]() __attribute__((always_inline)) {
@@ -504,13 +510,24 @@ __global__ __launch_bounds__(512, 2) void affine_qmm_tile_kernel(QmmMulti p, int
   // hold the chunk's groups (from the dword with the first one on: rows of an
   // odd number of groups start inside a dword), in two buffers. 64
   // consecutive dwords of a chunk's [scale, bias][128][ndw] are one copy.
+  // Sidecars that start on the second half of a dword are copied from that
+  // dword on (aligned, so never past what holds their first word) and counted
+  // from there: lead[] is 1 then.
+  uint32_t lead[2] = {0, 0};
+  if constexpr (!ALN) {
+    lead[0] = (uint32_t)(reinterpret_cast<uintptr_t>(sc) >> 1) & 1u;
+    lead[1] = (uint32_t)(reinterpret_cast<uintptr_t>(bi) >> 1) & 1u;
+    sc -= lead[0];
+    bi -= lead[1];
+  }
   const bool g32 = !GS64 && gs == 32;
   const int ndw = GS64 || g32 ? NDW : CS / 2 + 1;
   const uint32_t ldsa = lds0 + G::AUX0;
   // the last dword wholly inside the matrix; when the total is odd, the word
   // after it is copied alone (zero-extended)
-  const uint32_t atot = (uint32_t)N * ng * 2u, amax = (atot & ~3u) - 4u;
-  const bool odd = (atot & 2u) != 0 && bn0 + kTN >= N;
+  const uint32_t atot = (uint32_t)N * ng * 2u;
+  const bool odd = (ALN ? (atot & 2u) != 0 : ((atot ^ 2 * lead[0]) & 2u) != 0 || ((atot ^ 2 * lead[1]) & 2u) != 0) &&
+                   bn0 + kTN >= N;
   auto aux_chunk = [&](int c) __attribute__((always_inline)) {
     const int k = kb + 64 * CS * c;
     const uint32_t g0 = GS64 ? (uint32_t)k >> 6 : (uint32_t)k / (uint32_t)gs;
@@ -522,7 +539,8 @@ __global__ __launch_bounds__(512, 2) void affine_qmm_tile_kernel(QmmMulti p, int
       const bool bias = s >= per;
       const uint32_t d = 64 * (bias ? s - per : s) + lane;
       const uint32_t r = GS64 ? d / NDW : g32 ? d / NDW : d / (CS / 2 + 1);
-      const uint32_t u16i = ((uint32_t)min(bn0 + (int)r, N - 1) * ng + g0) & ~1u;
+      const uint32_t ld = bias ? lead[1] : lead[0], at = atot + 2 * ld, amax = (at & ~3u) - 4u;
+      const uint32_t u16i = ((uint32_t)min(bn0 + (int)r, N - 1) * ng + g0 + ld) & ~1u;
       const uint32_t o = 2 * u16i + 4 * (d - r * ndw);
       const uint16_t *src = bias ? bi : sc;
       const uint32_t dst = __builtin_amdgcn_readfirstlane(ldsa + (c & 1) * G::AB + 256 * s);
@@ -530,7 +548,7 @@ __global__ __launch_bounds__(512, 2) void affine_qmm_tile_kernel(QmmMulti p, int
         q_copy4(src, min(o, amax), dst);
       } else {
         // (waited for at once: its copies would not be the NA counted)
-        if (o == atot - 2) q_copy2(src, o, dst);
+        if (o == at - 2) q_copy2(src, o, dst);
         else q_copy4(src, min(o, amax), dst);
         q_wait<0>();
       }
@@ -545,7 +563,9 @@ __global__ __launch_bounds__(512, 2) void affine_qmm_tile_kernel(QmmMulti p, int
   for (int j = 0; j < 2; ++j) xrd[j] = smem + l32 * 128 + (((2 * run + j) ^ ((l32 >> 1) & 7)) << 4);
   const uint8_t *wrd = smem + NST * G::XB + nrow * G::RB;
   const uint8_t *ard = smem + G::AUX0 + nrow * (4 * ndw);
-  const int par = ((bn0 + nrow) * ng) & 1;
+  // word of a row's first group within its dword
+  const int pars = ((bn0 + nrow) * ng + (int)lead[0]) & 1;
+  const int parb = ALN ? pars : ((bn0 + nrow) * ng + (int)lead[1]) & 1;
   const int sh = BITS == 5 ? 16 * (run & 1) : 0;
 
   f32x16 acc[MI];
@@ -555,8 +575,11 @@ __global__ __launch_bounds__(512, 2) void affine_qmm_tile_kernel(QmmMulti p, int
   struct Raw {
     QRun<BITS> c;
     uint32_t s, b;
-    __device__ __forceinline__ float scale() const { return FP16 ? f16_to_f32(s) : bf16_to_f32(s); }
-    __device__ __forceinline__ float bias() const { return FP16 ? f16_to_f32(b) : bf16_to_f32(b); }
+  };
+  const int fp16 = p.fp16;
+  auto aux = [&](uint32_t v) __attribute__((always_inline)) {
+    if constexpr (ALN) return FP16 ? f16_to_f32(v) : bf16_to_f32(v);
+    else return aux_to_f32_sel(v, fp16);
   };
   // The next step's scale / bias words: GS64: two bytes on per step, and at a
   // chunk's first step to the other buffer and the word its first group
@@ -573,10 +596,11 @@ __global__ __launch_bounds__(512, 2) void affine_qmm_tile_kernel(QmmMulti p, int
   auto read_raw = [&](int wo, Raw &r) __attribute__((always_inline)) {
     const int c = rt / CS;
     if (rt == c * CS) cg0 = cgr;
-    const uint8_t *ap = ard + ((c & 1) * G::AB + 2 * (rgr - cg0)) + 2 * ((par + cg0) & 1);
+    const uint8_t *ap = ard + ((c & 1) * G::AB + 2 * (rgr - cg0));
+    const uint8_t *as = ap + 2 * ((pars + cg0) & 1), *ab = ALN ? as : ap + 2 * ((parb + cg0) & 1);
     r.c.read(wrd + wo, l32, run);
-    r.s = *reinterpret_cast<const uint16_t *>(ap);
-    r.b = *reinterpret_cast<const uint16_t *>(ap + kTN * 4 * ndw);
+    r.s = *reinterpret_cast<const uint16_t *>(as);
+    r.b = *reinterpret_cast<const uint16_t *>(ab + kTN * 4 * ndw);
     ++rt;
     if constexpr (GS64) {
       ++cgr;
@@ -623,7 +647,7 @@ __global__ __launch_bounds__(512, 2) void affine_qmm_tile_kernel(QmmMulti p, int
     uint32_t tw[3];
     raw.c.split(0, sh, tw);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) wf[0][i] = QRun<BITS>::pair(tw, 0, i, raw.scale(), raw.bias());
+    for (int i = 0; i < 4; ++i) wf[0][i] = QRun<BITS>::pair(tw, 0, i, aux(raw.s), aux(raw.b));
   }
   int so = 0, wo = 0, cs = 0;  // stages of step t; t % CS
   auto step = [&](auto copies, int t) __attribute__((always_inline)) {
@@ -652,7 +676,7 @@ __global__ __launch_bounds__(512, 2) void affine_qmm_tile_kernel(QmmMulti p, int
         if (i == P0) r.c.split(j ^ 1, sh, tw);
 #pragma unroll
         for (int q = 0; q < 4; ++q)
-          if (i == min(P0 + q, MI - 1)) wf[j ^ 1][q] = QRun<BITS>::pair(tw, j ^ 1, q, r.scale(), r.bias());
+          if (i == min(P0 + q, MI - 1)) wf[j ^ 1][q] = QRun<BITS>::pair(tw, j ^ 1, q, aux(r.s), aux(r.b));
         if constexpr (COPY) {
 #pragma unroll
           for (int c = 0; c < G::L; ++c)
@@ -846,22 +870,25 @@ bool affine_qmm_supported(const DevMat &m) {
   return true;
 }
 
-// The tile kernel: every matrix supported, the same K / bits / group size /
-// aux type, 16-byte copies of the packed rows (5-bit rows: 4-byte ones) and
-// per-lane offsets within a tile that fit 32 bits.
-static bool qmm_tile_ok(const DevMat *ms, int n, int x_stride) {
-  if (n < 1 || n > kQMultiMax || x_stride > (1 << 22)) return false;
+// Whether the tile kernel takes the product: every matrix supported, the same
+// K / bits / group size / aux type and per-lane offsets within a tile that fit
+// 32 bits; kQAligned: with 16-byte copies of the packed rows (5-bit rows: 4-byte
+// ones) and sidecars on whole dwords, kQDword: by dwords.
+enum { kQNone, kQAligned, kQDword };
+static int qmm_tile_form(const DevMat *ms, int n, int x_stride) {
+  if (n < 1 || n > kQMultiMax || x_stride > (1 << 22)) return kQNone;
+  int form = kQAligned;
   for (int i = 0; i < n; ++i) {
     const DevMat &m = ms[i];
-    if (!affine_qmm_supported(m)) return false;
-    if (m.I != ms[0].I || m.bits != ms[0].bits || m.gs != ms[0].gs || m.fp16 != ms[0].fp16) return false;
-    if (m.bits != 5 && (reinterpret_cast<uintptr_t>(m.w) & 15) != 0) return false;
-    if (m.row_bytes > (1 << 23) || (long long)m.O * m.ng > 0x7fff0000LL / 2) return false;
-    // scale / bias rows are copied by dwords
-    if (((reinterpret_cast<uintptr_t>(m.sc) | reinterpret_cast<uintptr_t>(m.bi)) & 3) != 0) return false;
-    if ((long long)m.O * m.ng < 2) return false;
+    if (!affine_qmm_supported(m)) return kQNone;
+    if (m.I != ms[0].I || m.bits != ms[0].bits || m.gs != ms[0].gs || m.fp16 != ms[0].fp16) return kQNone;
+    if (m.row_bytes > (1 << 23) || (long long)m.O * m.ng > 0x7fff0000LL / 2) return kQNone;
+    if ((long long)m.O * m.ng < 2) return kQNone;
+    const uintptr_t aux = reinterpret_cast<uintptr_t>(m.sc) | reinterpret_cast<uintptr_t>(m.bi);
+    if ((aux & 1) != 0) return kQNone;
+    if ((m.bits != 5 && (reinterpret_cast<uintptr_t>(m.w) & 15) != 0) || (aux & 3) != 0) form = kQDword;
   }
-  return true;
+  return form;
 }
 
 // Tile rows and K split of a product: the least estimated time in us. The
@@ -874,12 +901,13 @@ static bool qmm_tile_ok(const DevMat *ms, int n, int x_stride) {
 struct QmmPlan {
   int bm, split;
 };
-static QmmPlan qmm_plan(int M, int tiles, int cols, int ksteps, int bits) {
+static QmmPlan qmm_plan(int M, int tiles, int cols, int ksteps, int bits, int max_bm) {
   static const int kBm[5] = {32, 64, 128, 192, 256};
   QmmPlan best{256, 1};
   float tb = 1e30f;
   for (int c = 0; c < 5; ++c) {
     const int bm = kBm[c], mt = (M + bm - 1) / bm;
+    if (bm > max_bm) break;
     const float step = std::max(0.39f + 0.32f * bm / 256, 0.33f * bits / 8);
     const float fixed = 1.8f + 5.0f * bm / 256;
     for (int sp = 1; sp <= 16; ++sp) {
@@ -898,15 +926,64 @@ static QmmPlan qmm_plan(int M, int tiles, int cols, int ksteps, int bits) {
   return best;
 }
 
-template <int BITS, bool GS64, bool FP16>
+// the route of a product: kernel (kQNone: affine_qmm_kernel, one launch per
+// matrix, whose K split launch_affine_qmm chooses), tile rows and k ranges
+struct QmmRoute {
+  int form, bm, split;
+};
+static QmmRoute qmm_route(const DevMat *ms, int n, int x_stride, int M) {
+  // Products this small are launch and latency: the tile kernel's prologue (its
+  // rings, three or more steps ahead) and sum exchange cost more than they
+  // save. us, 64 x 64 kernel / tile kernel, 4-bit: 17 x 512 (M x N), K 2048:
+  // 8.0 / 9.0; 17 x 4096, K 2048: 10.6 / 11.1; 64 x 1024, K 2048: 10.3 / 10.3;
+  // 64 x 2048, K 2048: 13.6 / 11.9; 17 x 1024, K 9728: 13.2 / 13.7;
+  // 17 x 2048, K 9728: 16.2 / 14.4.
+  const bool small = n == 1 && (long long)M * ms[0].O <= (M <= 24 ? 81920 : 65536) &&
+                     (long long)ms[0].O * ms[0].I <= (10 << 20);
+  // By dwords above 64 rows only: up to there the 64 x 64 kernel forms every
+  // weight once as well. 4096 x 4096, 8-bit, 64 x 64 kernel / tile kernel by
+  // dwords, us: sidecars off 4 bytes, M 100: 29.5 / 20.7, 512: 81.9 / 37.3,
+  // 2048: 286 / 74; 4-bit weights off 16 bytes: 30.2 / 22.1, 79.8 / 36.0, 281 / 74.
+  const int form = small ? kQNone : qmm_tile_form(ms, n, x_stride);
+  if (form == kQNone || (form == kQDword && M <= kTile)) return QmmRoute{kQNone, 0, 0};
+  int tiles = 0, cols = 0;
+  for (int i = 0; i < n; ++i) {
+    tiles += (ms[i].O + kTN - 1) / kTN;
+    cols += (ms[i].O + 3) & ~3;
+  }
+  // (256 rows of 8-bit dwords leave no room for chunks of 32-code groups that
+  // start inside a dword)
+  const int max_bm = form == kQDword && ms[0].bits == 8 && ms[0].gs != 64 ? 192 : 256;
+  const QmmPlan plan = qmm_plan(M, tiles, cols, ms[0].I / 64, ms[0].bits, max_bm);
+  return QmmRoute{form, plan.bm, plan.split};
+}
+
+bool affine_qmm_route(const DevMat *ms, int n, int x_stride, int M, int (&route)[3]) {
+  for (int i = 0; i < n; ++i)
+    if (!affine_qmm_supported(ms[i])) return false;
+  const QmmRoute r = qmm_route(ms, n, x_stride, M);
+  route[0] = r.form;
+  route[1] = r.bm;
+  route[2] = r.split;
+  return true;
+}
+
+template <int BITS, bool GS64, bool FP16, bool ALN>
 static hipError_t launch_qmm_tile_bits(const QmmMulti &p, int bm, int mt, int tiles, int split, int ksteps,
                                        int slot, hipStream_t st) {
   const dim3 grid((mt * tiles * split + 7) / 8 * 8), block(512);
   switch (bm) {
-#define LH_QTILE(MI)                                                                                      \
-  case 32 * MI: hipLaunchKernelGGL((affine_qmm_tile_kernel<BITS, MI, GS64, FP16>), grid, block, 0, st, p, \
+#define LH_QTILE(MI)                                                                                           \
+  case 32 * MI: hipLaunchKernelGGL((affine_qmm_tile_kernel<BITS, MI, GS64, FP16, ALN>), grid, block, 0, st, p, \
                                    mt, tiles, ksteps, slot); break;
-    LH_QTILE(1) LH_QTILE(2) LH_QTILE(4) LH_QTILE(6) LH_QTILE(8)
+    LH_QTILE(1) LH_QTILE(2) LH_QTILE(4) LH_QTILE(6)
+    case 256:
+      if constexpr (ALN || GS64 || BITS != 8) {
+        hipLaunchKernelGGL((affine_qmm_tile_kernel<BITS, 8, GS64, FP16, ALN>), grid, block, 0, st, p, mt, tiles,
+                           ksteps, slot);
+        break;
+      }
+      return hipErrorInvalidValue;
 #undef LH_QTILE
     default: return hipErrorInvalidValue;
   }
@@ -914,7 +991,8 @@ static hipError_t launch_qmm_tile_bits(const QmmMulti &p, int bm, int mt, int ti
 }
 
 static hipError_t launch_qmm_tile(const DevMat *ms, int n, const uint16_t *x, int x_stride, int M,
-                                  void *const *ys, const int *y_strides, int y_bf16, hipStream_t st) {
+                                  void *const *ys, const int *y_strides, int y_bf16, const QmmRoute &route,
+                                  hipStream_t st) {
   QmmMulti p;
   p.x = x;
   p.n = n;
@@ -946,10 +1024,8 @@ static hipError_t launch_qmm_tile(const DevMat *ms, int n, const uint16_t *x, in
   }
   p.vec = yv ? 1 : 0;
   const int ksteps_all = p.K / 64;
-  const QmmPlan plan = qmm_plan(M, tiles, cols, ksteps_all, ms[0].bits);
-  const int mt = (M + plan.bm - 1) / plan.bm;
-  const int ksteps = (ksteps_all + plan.split - 1) / plan.split;
-  const int split = plan.split;
+  const int bm = route.bm, split = route.split, mt = (M + bm - 1) / bm;
+  const int ksteps = (ksteps_all + split - 1) / split;
   SlotRing::Lease lease;
   if (split > 1) {
     const hipError_t le = g_qmm_slots.take(st, lease);
@@ -958,15 +1034,15 @@ static hipError_t launch_qmm_tile(const DevMat *ms, int n, const uint16_t *x, in
   const int slot = split > 1 ? lease.slot() : -1;
   hipError_t e;
   switch (ms[0].bits) {
-#define LH_QBITS(B)                                                                                     \
-  case B:                                                                                               \
-    e = p.gs == 64 ? (p.fp16 ? launch_qmm_tile_bits<B, true, true>(p, plan.bm, mt, tiles, split, ksteps, slot, st)     \
-                             : launch_qmm_tile_bits<B, true, false>(p, plan.bm, mt, tiles, split, ksteps, slot, st))   \
-                   : (p.fp16 ? launch_qmm_tile_bits<B, false, true>(p, plan.bm, mt, tiles, split, ksteps, slot, st)    \
-                             : launch_qmm_tile_bits<B, false, false>(p, plan.bm, mt, tiles, split, ksteps, slot, st)); \
-    break;
+#define LH_QFORM(B, G64)                                                                                         \
+  (route.form == kQDword ? launch_qmm_tile_bits<B, G64, false, false>(p, bm, mt, tiles, split, ksteps, slot, st) \
+   : p.fp16              ? launch_qmm_tile_bits<B, G64, true, true>(p, bm, mt, tiles, split, ksteps, slot, st)   \
+                         : launch_qmm_tile_bits<B, G64, false, true>(p, bm, mt, tiles, split, ksteps, slot, st))
+#define LH_QBITS(B) \
+  case B: e = p.gs == 64 ? LH_QFORM(B, true) : LH_QFORM(B, false); break;
     LH_QBITS(4) LH_QBITS(5) LH_QBITS(6) LH_QBITS(8)
 #undef LH_QBITS
+#undef LH_QFORM
     default: return hipErrorInvalidValue;
   }
   if (e != hipSuccess || split == 1) return e;
@@ -982,7 +1058,10 @@ hipError_t launch_affine_qmm_multi(const DevMat *ms, int n, const uint16_t *x, i
   if ((reinterpret_cast<uintptr_t>(x) & 15) != 0 || (x_stride & 7) != 0) return hipErrorInvalidValue;
   int strides[kQMultiMax];
   for (int i = 0; i < n; ++i) strides[i] = ms[i].O;
-  if (n > 1 && qmm_tile_ok(ms, n, x_stride)) return launch_qmm_tile(ms, n, x, x_stride, M, ys, strides, y_bf16, st);
+  if (n > 1) {
+    const QmmRoute r = qmm_route(ms, n, x_stride, M);
+    if (r.form != kQNone) return launch_qmm_tile(ms, n, x, x_stride, M, ys, strides, y_bf16, r, st);
+  }
   for (int i = 0; i < n; ++i) {
     const hipError_t e = launch_affine_qmm(ms[i], x, x_stride, M, ys[i], ms[i].O, y_bf16, st);
     if (e != hipSuccess) return e;
@@ -994,17 +1073,11 @@ hipError_t launch_affine_qmm(const DevMat &m, const uint16_t *x, int x_stride, i
                              int y_stride, int y_bf16, hipStream_t st) {
   if (!affine_qmm_supported(m) || M <= 0) return hipErrorInvalidValue;
   if ((reinterpret_cast<uintptr_t>(x) & 15) != 0 || (x_stride & 7) != 0) return hipErrorInvalidValue;
-  // Products this small are launch and latency: the tile kernel's prologue (its
-  // rings, three or more steps ahead) and sum exchange cost more than they
-  // save. us, 64 x 64 kernel / tile kernel, 4-bit: 17 x 512 (M x N), K 2048:
-  // 8.0 / 9.0; 17 x 4096, K 2048: 10.6 / 11.1; 64 x 1024, K 2048: 10.3 / 10.3;
-  // 64 x 2048, K 2048: 13.6 / 11.9; 17 x 1024, K 9728: 13.2 / 13.7;
-  // 17 x 2048, K 9728: 16.2 / 14.4.
-  const bool small = (long long)M * m.O <= (M <= 24 ? 81920 : 65536) && (long long)m.O * m.I <= (10 << 20);
-  if (!small && qmm_tile_ok(&m, 1, x_stride)) {
+  const QmmRoute r = qmm_route(&m, 1, x_stride, M);
+  if (r.form != kQNone) {
     void *ys[1] = {y};
     const int strides[1] = {y_stride};
-    return launch_qmm_tile(&m, 1, x, x_stride, M, ys, strides, y_bf16, st);
+    return launch_qmm_tile(&m, 1, x, x_stride, M, ys, strides, y_bf16, r, st);
   }
   GemmParams p;
   p.w = m.w;

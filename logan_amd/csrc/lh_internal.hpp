@@ -107,6 +107,8 @@ hipError_t launch_hilo_join(const HiloBatch &b, hipStream_t st);
 hipError_t launch_affine_qmm(const DevMat &m, const uint16_t *x, int x_stride, int M, void *y,
                              int y_stride, int y_bf16, hipStream_t st);
 bool affine_qmm_supported(const DevMat &m);
+// {0 (64 x 64 tiles) | 1 (tile kernel) | 2 (its dword form), tile rows, k ranges}
+bool affine_qmm_route(const DevMat *ms, int n, int x_stride, int M, int (&route)[3]);
 // up to 8 matrices sharing x (same I, bits, group size, aux type) in one
 // grid where the tile kernel applies, else one launch per matrix; ys[i] is
 // [M][O_i]

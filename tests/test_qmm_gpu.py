@@ -31,6 +31,17 @@ def dev_matrix(torch, w, sc, bi, O, I, bits, gs, fp16=False):
                         to_dev(bi.view(np.int16), torch), O, I, bits, gs, fp16)
 
 
+def qmm_route(mats, M):
+    """(form, tile rows, k ranges) that the library gives these matrices."""
+    import ctypes as C
+    from logan_amd import _lib as L
+
+    arr = (L.Affine * len(mats))(*[m.c() for m in mats])
+    r = (C.c_int * 3)()
+    assert L.lib().logan_hip_affine_qmm_route(arr, len(mats), M, mats[0].I, r) == 1
+    return tuple(r)
+
+
 CASES = [
     # (M, O, I, bits, gs, fp16): tile edges in M and O, every width, group sizes
     (1, 64, 64, 4, 64, False),
@@ -316,3 +327,60 @@ def test_qmm_tile_edges(gpu, M, O, I, bits, gs, fp16):
     m4 = AffineMatrix(off.view(m.weights.shape), m.scales, m.biases, O, I, bits, gs, fp16)
     y4 = affine_qmm(m4, x, out_dtype=torch.float32)
     assert normwise_rel(y4.cpu().numpy(), ref) <= 1e-5
+
+
+def shifted(torch, t, nbytes):
+    """A copy of t that starts nbytes past an aligned address and ends with its buffer."""
+    flat = t.contiguous().view(torch.uint8).reshape(-1)
+    buf = torch.empty(nbytes + flat.numel(), dtype=torch.uint8, device=t.device)
+    buf[nbytes:].copy_(flat)
+    return buf[nbytes:].view(t.dtype).view(t.shape)
+
+
+ALIGN_CASES = [
+    # (M, O, I, bits, gs, fp16): odd and even numbers of groups per row (and in
+    # all), every group form, one and several k ranges, chunks of scale words
+    # that end early
+    (65, 1033, 192, 4, 64, False),
+    (130, 2880, 2880, 8, 64, False),
+    (300, 4096, 1152, 6, 192, True),
+    (700, 4090, 448, 5, 64, True),
+    (2000, 4090, 320, 8, 64, True),
+    (1999, 4100, 256, 8, 32, False),
+    (1500, 4090, 1088, 4, 32, True),
+    (520, 4001, 2880, 5, 96, False),
+    (270, 515, 2048, 6, 32, False),
+]
+
+
+@pytest.mark.parametrize("M,O,I,bits,gs,fp16", ALIGN_CASES, ids=lambda v: str(v))
+def test_qmm_operand_alignment(gpu, M, O, I, bits, gs, fp16):
+    """Weights off 16 bytes and sidecars on the second half of a dword, each
+    alone and together: the tile kernel, with the bits of the aligned call
+    where the tiles are the same, else (and for it) within 1e-5 of the oracle on
+    a sample of columns."""
+    import torch
+    from logan_amd.device import AffineMatrix, affine_qmm
+
+    print(f"qmm align M={M} O={O} I={I} bits={bits} gs={gs}", flush=True)
+    rng = np.random.default_rng(M + O + bits)
+    w, sc, bi = make_affine(rng, O, I, bits, gs, fp16)
+    xb = make_x(rng, M, I).reshape(M, I)
+    x = to_dev(xb.view(np.int16), torch).view(torch.bfloat16)
+    m = dev_matrix(torch, w, sc, bi, O, I, bits, gs, fp16)
+    y = affine_qmm(m, x, out_dtype=torch.float32)
+    cols = np.unique(np.concatenate([np.arange(0, O, max(1, O // 24)), np.arange(O - 5, O)]))
+    ng = I // gs
+    ref = oracle.affine_qmm_bf16(bf16_to_f32(xb).reshape(M, I), w.reshape(O, -1)[cols],
+                                 sc.reshape(O, ng)[cols].reshape(-1), bi.reshape(O, ng)[cols].reshape(-1),
+                                 len(cols), I, bits, gs, fp16)
+    assert normwise_rel(y.cpu().numpy()[:, cols], ref) <= 1e-5
+    for ow, os_, ob in ((4, 0, 0), (12, 2, 2), (0, 2, 2), (0, 2, 0), (8, 0, 2)):
+        ms = AffineMatrix(shifted(torch, m.weights, ow), shifted(torch, m.scales, os_),
+                          shifted(torch, m.biases, ob), O, I, bits, gs, fp16)
+        want = 1 if bits == 5 and os_ == ob == 0 else 2
+        assert qmm_route([ms], M)[0] == want
+        ys = affine_qmm(ms, x, out_dtype=torch.float32)
+        if qmm_route([ms], M)[1:] == qmm_route([m], M)[1:]:
+            assert torch.equal(ys, y), (ow, os_, ob)
+        assert normwise_rel(ys.cpu().numpy()[:, cols], ref) <= 1e-5, (ow, os_, ob)
