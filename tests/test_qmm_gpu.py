@@ -52,7 +52,7 @@ CASES = [
     (64, 512, 2048, 4, 64, False),   # config-5 attention projection shape, one tile of M
     (33, 192, 1024, 5, 32, True),
     (65, 130, 512, 8, 128, False),
-    (200, 96, 320, 5, 64, False),    # large-tile kernel: M > 64, partial tiles in M and N
+    (200, 96, 320, 5, 64, False),    # M > 64, partial tiles in M and N
     (300, 257, 128, 4, 32, True),
 ]
 
@@ -99,9 +99,9 @@ def test_qmm_prefill_chunk(gpu):
 
 @pytest.mark.parametrize("bits,gs,fp16", [(4, 64, False), (5, 64, True), (8, 128, False)])
 def test_qmm_large_tiles_ragged(gpu, bits, gs, fp16):
-    """A grid of >= 192 tiles of 128 x 128 (the large-tile kernel) with
-    partial tiles in both M and N, against the oracle on a sample of output
-    columns (every column of the last, partial tile included)."""
+    """50 column tiles of the tile kernel, partial tiles in both M and N,
+    against the oracle on a sample of output columns (every column of the
+    last, partial tile included)."""
     import torch
     from logan_amd.device import affine_qmm
 
@@ -149,9 +149,8 @@ def test_qmm_leaves_outside_untouched(gpu):
                          ids=["ba", "k_v", "o_out", "q"])
 def test_qmm_config5_prefill_projections(gpu, O, I):
     """The config-5 projections at the prefill chunk M = 512: grids with few
-    tiles split K (ordered f32 partials and a reduction launch), large grids
-    take the double-buffered 128 x 128 kernel. Sampled output columns against
-    the oracle; two calls give identical bits."""
+    tiles split K (ordered f32 partials and a reduction launch). Sampled
+    output columns against the oracle; two calls give identical bits."""
     import torch
     from logan_amd.device import affine_qmm
 
@@ -184,14 +183,13 @@ MULTI_CASES = [
     (300, [100, 257, 64], 192, 5, 64, True),       # ragged tiles, 5-bit runs at bit 16
     (256, [130, 72], 512, 6, 128, False),
     (384, [200, 96, 40, 33], 256, 8, 32, False),
-    (270, [96, 64], 192, 4, 96, False),            # group size 96: one launch per matrix
-    (64, [128, 96], 256, 4, 64, False),            # M < 256: one launch per matrix
+    (270, [96, 64], 192, 4, 96, False),            # group size 96
+    (64, [128, 96], 256, 4, 64, False),            # few rows, in one grid too
 ]
 
 
 KSLAB_CASES = [
-    # grids short of 192 tiles of 256 x 128 with K a multiple of 1024: 64 x 64
-    # tiles, K split across the 8 waves of a block (2, 4 or 6 steps per wave)
+    # grids with few tiles and a long K: several k ranges
     (300, [2048], 1024, 5, 32, True),
     (270, [200, 130], 2048, 6, 128, False),        # ragged N and M
     (511, [1000], 3072, 8, 64, False),
@@ -282,11 +280,67 @@ def test_split_qmm_on_three_overlapping_streams(gpu):
         assert normwise_rel(serial[s].cpu().numpy()[:, cols], ref) <= 1e-5
 
 
+def test_split_tile_products_on_overlapping_streams(gpu):
+    """The two kernels with K split lay their partial sums out differently in
+    the same 2 slots: tile products of one and of several matrices and a 64 x
+    64 one, back to back on each of three streams with no synchronisation
+    between them. Every output equals the single-stream result bitwise; the
+    serial results against the oracle on a sample of columns."""
+    import torch
+    from logan_amd.device import affine_qmm, affine_qmm_multi
+
+    # (M, Os, I, bits), all split: one matrix, several, and the 64 x 64 kernel
+    jobs = [(512, (512,), 2048, 4), (270, (200, 130), 2048, 6), (64, (512,), 4096, 4)]
+    sets, serial = [], []
+    for s in range(3):
+        rng = np.random.default_rng(950 + s)
+        row = []
+        for M, Os, I, bits in jobs:
+            mats = [make_affine(rng, O, I, bits, 64) for O in Os]
+            dev = [dev_matrix(torch, *m, O, I, bits, 64) for m, O in zip(mats, Os)]
+            xb = make_x(rng, M, I).reshape(M, I)
+            x = to_dev(xb.view(np.int16), torch).view(torch.bfloat16)
+            form, _, split = qmm_route(dev, M)
+            assert (form == 1 and split > 1) if M > 64 else form == 0
+            row.append((dev, x, mats, xb))
+        sets.append(row)
+        serial.append([affine_qmm_multi(dev, x, out_dtype=torch.float32) if len(dev) > 1
+                       else [affine_qmm(dev[0], x, out_dtype=torch.float32)] for dev, x, _, _ in row])
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    outs = [[[[torch.full_like(y, float("nan")) for y in ys] for ys in serial[s]] for _ in range(4)]
+            for s in range(3)]
+    torch.cuda.synchronize()
+    for r in range(4):
+        for s in range(3):
+            with torch.cuda.stream(streams[s]):
+                for i in range(3):
+                    dev, x, _, _ = sets[s][(i + s) % 3]
+                    ys = outs[s][r][(i + s) % 3]
+                    if len(dev) > 1:
+                        affine_qmm_multi(dev, x, outs=ys, stream=streams[s])
+                    else:
+                        affine_qmm(dev[0], x, out=ys[0], stream=streams[s])
+    torch.cuda.synchronize()
+    for s in range(3):
+        for r in range(4):
+            for ys, want in zip(outs[s][r], serial[s]):
+                assert all(torch.equal(a, b) for a, b in zip(ys, want)), (s, r)
+        for (M, Os, I, bits), (_, _, mats, xb), ys in zip(jobs, sets[s], serial[s]):
+            for (w, sc, bi), O, y in zip(mats, Os, ys):
+                cols = np.arange(0, O, 37)
+                ng = I // 64
+                ref = oracle.affine_qmm_bf16(bf16_to_f32(xb).reshape(M, I), w.reshape(O, -1)[cols],
+                                             sc.reshape(O, ng)[cols].reshape(-1),
+                                             bi.reshape(O, ng)[cols].reshape(-1), len(cols), I, bits, 64)
+                assert normwise_rel(y.cpu().numpy()[:, cols], ref) <= 1e-5
+
+
 TILE_CASES = [
-    # (M, O, I, bits, gs, fp16): rows at the edges of the 32 / 64 / 128 / 192 /
-    # 256-row tiles; 1, 2, 3, 5, 9, 45 steps of 64 codes (pipelines that never
-    # fill, chunks of scale words that end early); rows of an odd number of
-    # groups, which start inside a dword; group sizes 32 to 192
+    # (M, O, I, bits, gs, fp16): rows at the edges of the tiles; 1, 2, 3, 5, 9,
+    # 45 steps of 64 codes (pipelines that never fill, chunks of scale words that
+    # end early); rows of an odd number of groups, which start inside a dword;
+    # group sizes 32 to 192
     (31, 130, 64, 8, 64, False),
     (33, 257, 128, 4, 32, True),
     (65, 96, 192, 6, 64, False),
@@ -307,26 +361,32 @@ TILE_CASES = [
 
 @pytest.mark.parametrize("M,O,I,bits,gs,fp16", TILE_CASES, ids=lambda v: str(v))
 def test_qmm_tile_edges(gpu, M, O, I, bits, gs, fp16):
-    """Every column against the oracle at shapes where tiles, pipelines and
-    scale rows end unevenly, weights at a 16-byte and at a 4-byte offset (the
-    64 x 64 kernel), the two within f32 rounding of each other."""
+    """Shapes where tiles, pipelines and scale rows end unevenly: alone (most
+    are small enough for the 64 x 64 kernel) and as the second of two matrices,
+    which the tile kernel always takes. Every column of both against the
+    oracle, and the two calls against each other (f32 sums in another order)."""
     import torch
-    from logan_amd.device import AffineMatrix, affine_qmm
+    from logan_amd.device import affine_qmm, affine_qmm_multi
 
     rng = np.random.default_rng(M * 7 + O + bits)
     w, sc, bi = make_affine(rng, O, I, bits, gs, fp16)
     xb = make_x(rng, M, I).reshape(M, I)
     x = to_dev(xb.view(np.int16), torch).view(torch.bfloat16)
-    ref = oracle.affine_qmm_bf16(bf16_to_f32(xb).reshape(M, I), w, sc, bi, O, I, bits, gs, fp16)
+    xf = bf16_to_f32(xb).reshape(M, I)
+    ref = oracle.affine_qmm_bf16(xf, w, sc, bi, O, I, bits, gs, fp16)
     m = dev_matrix(torch, w, sc, bi, O, I, bits, gs, fp16)
     y = affine_qmm(m, x, out_dtype=torch.float32)
     assert normwise_rel(y.cpu().numpy(), ref) <= 1e-5
-    buf = torch.empty(w.size + 16, dtype=torch.uint8, device="cuda")
-    off = buf[4:4 + w.size]
-    off.copy_(m.weights.reshape(-1))
-    m4 = AffineMatrix(off.view(m.weights.shape), m.scales, m.biases, O, I, bits, gs, fp16)
-    y4 = affine_qmm(m4, x, out_dtype=torch.float32)
-    assert normwise_rel(y4.cpu().numpy(), ref) <= 1e-5
+    O2 = 37
+    w2, sc2, bi2 = make_affine(rng, O2, I, bits, gs, fp16)
+    mats = [dev_matrix(torch, w2, sc2, bi2, O2, I, bits, gs, fp16), m]
+    assert qmm_route(mats, M)[0] == 1
+    assert qmm_route([m], M)[0] == (0 if M * O <= 65536 else 1)
+    y2, yt = affine_qmm_multi(mats, x, out_dtype=torch.float32)
+    assert normwise_rel(yt.cpu().numpy(), ref) <= 1e-5
+    ref2 = oracle.affine_qmm_bf16(xf, w2, sc2, bi2, O2, I, bits, gs, fp16)
+    assert normwise_rel(y2.cpu().numpy(), ref2) <= 1e-5
+    assert normwise_rel(yt.cpu().numpy(), y.cpu().numpy()) <= 1e-5
 
 
 def shifted(torch, t, nbytes):
@@ -384,3 +444,83 @@ def test_qmm_operand_alignment(gpu, M, O, I, bits, gs, fp16):
         if qmm_route([ms], M)[1:] == qmm_route([m], M)[1:]:
             assert torch.equal(ys, y), (ow, os_, ob)
         assert normwise_rel(ys.cpu().numpy()[:, cols], ref) <= 1e-5, (ow, os_, ob)
+
+
+# Sizes that give each tile height its one k range: (rows, M) with 32 column
+# tiles, M short of whole tiles
+TILE_ROWS = [(32, 250), (64, 500), (128, 1000), (192, 1500), (256, 2000)]
+TILE_OS = (3901, 77)  # ragged column tiles, odd totals of groups where a row has an odd number
+# (I, gs, fp16, bytes off alignment of weights, scales, biases): 1 to 17 steps of
+# 64 codes (pipelines that never fill, chunks of scale words that end early),
+# every group form and aux type; then the dword form
+TILE_KINDS = [(64, 64, False, None), (128, 64, True, None), (192, 64, False, None), (576, 64, True, None),
+              (1088, 64, False, None), (128, 32, True, None), (320, 32, False, None), (1088, 32, True, None),
+              (192, 96, True, None), (576, 192, False, None),
+              (576, 64, True, (4, 2, 2)), (1088, 64, False, (8, 2, 0)), (320, 32, True, (4, 0, 2)),
+              (576, 192, False, (12, 2, 2)), (1088, 32, False, (4, 2, 2))]
+
+
+def tile_rows(rows, bits, gs, off):
+    """256 rows of 8-bit dwords exist for groups of 64 only."""
+    return 128 if rows == 256 and bits == 8 and gs != 64 and off else rows
+
+
+def weights64(torch, m):
+    """bf16(code * scale + bias) of a device matrix, in float64."""
+    at = torch.arange(m.I, device="cuda") * m.bits
+    w = m.weights.reshape(m.O, -1).int()
+    lo = at // 8
+    c = ((w[:, lo] | (w[:, torch.clamp(lo + 1, max=w.shape[1] - 1)] << 8)) >> (at % 8).int()) & ((1 << m.bits) - 1)
+    t = torch.float16 if m.aux_fp16 else torch.bfloat16
+    s, b = (p.reshape(m.O, -1).view(t).double().repeat_interleave(m.group_size, 1) for p in (m.scales, m.biases))
+    return (c.double() * s + b).float().to(torch.bfloat16).double()
+
+
+@pytest.mark.parametrize("bits", [4, 5, 6, 8])
+@pytest.mark.parametrize("rows,M", TILE_ROWS)
+def test_qmm_tile_forms(gpu, rows, M, bits):
+    """Every form of the tile kernel: two matrices in one grid against float64
+    (sums of at most 1088 products in f32, another order: 1e-5 of the largest),
+    bf16 outputs the RNE of the f32 ones; one matrix into rows of an odd stride
+    (element stores), nothing past its columns; and a part of it on the 64 x 64
+    kernel."""
+    import ctypes as C
+
+    import torch
+    from logan_amd import _lib as L
+    from logan_amd.device import AffineMatrix, affine_qmm, affine_qmm_multi
+
+    for I, gs, fp16, off in TILE_KINDS:
+        print(f"qmm tile rows={rows} M={M} bits={bits} I={I} gs={gs} off={off}", flush=True)
+        rng = np.random.default_rng(rows + bits * I + gs)
+        mats = []
+        for O in TILE_OS:
+            m = dev_matrix(torch, *make_affine(rng, O, I, bits, gs, fp16), O, I, bits, gs, fp16)
+            if off:
+                m = AffineMatrix(shifted(torch, m.weights, off[0]), shifted(torch, m.scales, off[1]),
+                                 shifted(torch, m.biases, off[2]), O, I, bits, gs, fp16)
+            mats.append(m)
+        x = to_dev(make_x(rng, M, I).reshape(M, I).view(np.int16), torch).view(torch.bfloat16)
+        want = (2 if off else 1, tile_rows(rows, bits, gs, off), 1)
+        assert qmm_route(mats, M) == want
+        ys = affine_qmm_multi(mats, x, out_dtype=torch.float32)
+        ybs = affine_qmm_multi(mats, x, out_dtype=torch.bfloat16)
+        for m, y, yb in zip(mats, ys, ybs):
+            ref = x.double() @ weights64(torch, m).T.contiguous()
+            assert float((y.double() - ref).abs().max() / ref.abs().max()) <= 1e-5, m.O
+            assert torch.equal(yb, y.to(torch.bfloat16))
+        m, y = mats[0], ys[0]
+        assert qmm_route([m], M) == want
+        for dt, yd in ((torch.float32, L.LOGAN_HIP_F32), (torch.bfloat16, L.LOGAN_HIP_BF16)):
+            wide = torch.full((M, m.O + 2), 7.0, dtype=dt, device="cuda")
+            a = m.c()
+            rc = L.lib().logan_hip_affine_qmm(C.byref(a), x.data_ptr(), M, I, wide.data_ptr(), m.O + 2, yd, None)
+            torch.cuda.synchronize()
+            assert rc == 1
+            assert torch.equal(wide[:, :m.O], y.to(dt)) and torch.all(wide[:, m.O:] == 7.0)
+        n = 1000
+        part = AffineMatrix(m.weights[:n], m.scales.reshape(m.O, -1)[:n], m.biases.reshape(m.O, -1)[:n], n, I, bits,
+                            gs, fp16)
+        assert qmm_route([part], 64)[0] == 0
+        y64 = affine_qmm(part, x[:64], out_dtype=torch.float32)
+        assert float((y64 - y[:64, :n]).abs().max() / y64.abs().max()) <= 1e-5

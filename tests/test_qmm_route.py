@@ -66,3 +66,21 @@ def test_routes_fit_the_launch():
     assert route(512, [4096], 4096, 8, 64, off=(0, 1, 0))[0] == 0
     assert route(512, [4096], 4096, 8, 64, off=(2, 0, 0)) is None
     assert route(512, [4096], 96, 8, 32) is None
+
+
+def test_tile_form_cases_reach_every_form():
+    """The device test's cases are routed to the tile kernel's every
+    instantiation: (bits, rows, 64-code groups or not, aux type, aligned) and
+    (bits, rows, groups) of the dword form."""
+    from test_qmm_gpu import TILE_KINDS, TILE_OS, TILE_ROWS, tile_rows
+
+    hit = set()
+    for bits in (4, 5, 6, 8):
+        for rows, M in TILE_ROWS:
+            for I, gs, fp16, off in TILE_KINDS:
+                r = route(M, TILE_OS, I, bits, gs, fp16, off or (0, 0, 0))
+                assert r == (2 if off else 1, tile_rows(rows, bits, gs, off), 1)
+                hit.add((bits, r[1], gs == 64, None if off else fp16))
+    want = {(b, r, g, t) for b in (4, 5, 6, 8) for r in (32, 64, 128, 192, 256) for g in (True, False)
+            for t in (True, False, None)} - {(8, 256, False, None)}
+    assert hit == want
