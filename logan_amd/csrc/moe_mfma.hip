@@ -274,6 +274,16 @@ __global__ __launch_bounds__(kMGroupThreads) void moe_mgroup_kernel(MoeArgs a, M
 #endif
 constexpr int kMGuSmallB = 128;
 
+// h = silu(gate) * up (logan-qwen4/src/lib.rs:8807-8809) as hi + lo bf16, lo the
+// rest of the exact product. The fma is written out: left to the compiler, one
+// of the wide form's unrolled places rounded the product first, and a slot's
+// result depended on its place in the tile (which varies from call to call).
+__device__ __forceinline__ void swiglu_hilo(float gate, float up, uint32_t &hi, uint32_t &lo) {
+  const float s = silu(gate);
+  hi = f32_to_bf16_rne(s * up);
+  lo = f32_to_bf16_rne(fmaf(s, up, -bf16_to_f32(hi)));
+}
+
 // scale/bias words of GU steps for one lane's row: with 64-code groups the GU
 // consecutive u16 come in one load
 template <int GU, bool GS64>
@@ -437,9 +447,8 @@ __global__ __launch_bounds__(WAVES * 64, WAVES <= 4 ? 2 : MOE_GU_MINW) void moe_
     for (int i = 0; i < 4; ++i) {
       const int m = 4 * g + i;
       if (m < cnt) {
-        const float h = silu(accg[i]) * accu[i];
-        const uint32_t hi = f32_to_bf16_rne(h);
-        const uint32_t lo = f32_to_bf16_rne(h - bf16_to_f32(hi));
+        uint32_t hi, lo;
+        swiglu_hilo(accg[i], accu[i], hi, lo);
         const size_t o = (size_t)(row0 + m) * hmax + S::op_pos(jj);
         w.h_hi[o] = (uint16_t)hi;
         w.h_lo[o] = (uint16_t)lo;
@@ -767,17 +776,15 @@ __global__ __launch_bounds__(512, 1) void moe_gateup_lds_kernel(MoeArgs a, MoeMW
         cs ^= 1;
       }
       if (c == nch - 1) {
-        // h = silu(gate) * up (logan-qwen4/src/lib.rs:8807-8809) as hi + lo
-        // bf16, each at its place in the down pass's operand order
+        // h's halves, each at its place in the down pass's operand order
         const int jj = jw0 + rg * RPB + r16;
         if (jj < rows) {
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
             const int m = 4 * g + i;
             if (m < cnt) {
-              const float h = silu(acc[0][i]) * acc[1][i];
-              const uint32_t hi = f32_to_bf16_rne(h);
-              const uint32_t lo = f32_to_bf16_rne(h - bf16_to_f32(hi));
+              uint32_t hi, lo;
+              swiglu_hilo(acc[0][i], acc[1][i], hi, lo);
               const size_t o = (size_t)(row0 + m) * hmax + S::op_pos(jj);
               w.h_hi[o] = (uint16_t)hi;
               w.h_lo[o] = (uint16_t)lo;
@@ -1001,9 +1008,8 @@ __device__ __forceinline__ void moe_gateup_wide_tile(const MoeArgs &a, const Moe
         for (int i = 0; i < 4; ++i) {
           const int m = 16 * t + 4 * g + i;
           if (m < cnt) {
-            const float h = silu(acc[rg][0][t][i]) * acc[rg][1][t][i];
-            const uint32_t hi = f32_to_bf16_rne(h);
-            const uint32_t lo = f32_to_bf16_rne(h - bf16_to_f32(hi));
+            uint32_t hi, lo;
+            swiglu_hilo(acc[rg][0][t][i], acc[rg][1][t][i], hi, lo);
             const size_t o = (size_t)(row0 + m) * hmax + S::op_pos(jj);
             w.h_hi[o] = (uint16_t)hi;
             w.h_lo[o] = (uint16_t)lo;

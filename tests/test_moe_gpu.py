@@ -538,6 +538,31 @@ def test_moe_prefill_wide_tiles(gpu, bits, fp16, E, k, B, D, inter, sinter):
         assert normwise_rel(out32[t], out_d[t]) <= 5e-5
 
 
+@pytest.mark.parametrize("bits,fp16,E,k,B,part,D,inter,sinter", [
+    (4, False, 64, 8, 801, 200, 2048, 512, 256), (4, True, 96, 16, 1600, 190, 768, 256, 512),
+    (8, False, 64, 8, 701, 200, 1024, 384, 512), (8, True, 64, 8, 1999, 250, 256, 128, 128),
+    (4, False, 48, 8, 801, 180, 4096, 512, 0)])
+def test_moe_wide_tiles_bits(gpu, bits, fp16, E, k, B, part, D, inter, sinter):
+    """A slot's place in its tile, which differs from call to call, and the
+    tile's form do not touch its bits: repeated calls of a batch on wide tiles
+    are equal, and equal to the batch in parts that take 16-slot tiles."""
+    import torch
+
+    print(f"moe wide bits bits={bits} fp16={fp16} E={E} B={B} D={D} inter={inter}", flush=True)
+    layer = Layer(torch, E, k, D, inter, bits, 64, seed=151 + bits + D, fp16=fp16, shared=sinter > 0,
+                  sinter=sinter or None)
+    rng = np.random.default_rng(152 + D)
+    xb = make_x(rng, B, D)
+    lb = make_logits(rng, B, E, zipf_s=1.1)
+    assert B * k >= 32 * E and part * k < 32 * E and part > 128
+    out = run_layer(torch, layer, xb, lb, torch.float32)[0]
+    for _ in range(3):
+        assert torch.equal(run_layer(torch, layer, xb, lb, torch.float32)[0], out)
+    for t in range(0, B - part + 1, part):
+        o = run_layer(torch, layer, xb[t:t + part], lb[t:t + part], torch.float32)[0]
+        assert torch.equal(o, out[t:t + part]), t
+
+
 @pytest.mark.parametrize("mfma_min_b", [1 << 20], indirect=True)
 def test_moe_large_batch_per_token_passes(gpu, mfma_min_b):
     """With the MFMA path off, B = 100 runs the per-token path in passes of
