@@ -232,10 +232,13 @@ static SlotRing g_qmm_slots(kQSlots);
 // Products of up to kQMultiMax matrices that read the same x (q/k/v, qkvz/ba,
 // gate/up) in one grid, BM x 128 output tiles, one 8-wave block per CU.
 //
-// What bounds it: 256-row tiles the vector and matrix pipes together (per
-// 64-k step and SIMD 1024 cycles of MFMA and about 600 issue cycles of VALU,
-// most of it the forming of the bf16 weights); tiles of at most 128 rows the
-// forming alone and, at 8 bits, the stream of codes from HBM. Hence:
+// What bounds it: 256-row tiles the matrix and vector pipes, which hardly
+// overlap (8-bit, 2 x 14336 columns, K 4096, M 2048: of 2,090 cycles per 64-k
+// step a SIMD's matrix pipe is busy 1,024 and its vector pipe 690, most of it
+// the forming of the bf16 weights, at the 1.8-1.86 GHz the card holds under this
+// load); tiles of at most 128 rows a step's chain of LDS reads, forming, MFMAs
+// and barrier with two waves a SIMD (M 100: 1,830 cycles for 512 and 510), the
+// codes arriving at 2.7 TB/s. Hence:
 //   * every copy from memory goes straight into LDS (global_load_lds, issued
 //     through inline assembly and waited for by count) NST - 1 steps ahead: x
 //     rows, packed codes, and the scale / bias words a chunk of steps at a
@@ -247,21 +250,26 @@ static SlotRing g_qmm_slots(kQSlots);
 //     waves of a tile add their sums through LDS after the last step;
 //   * the copies of a step are issued between its MFMAs, at the places the
 //     scheduling barriers fix: issued together at its start they hold the
-//     waves at the CU's one address path before their first MFMA (2 x 14336
-//     columns, 8-bit, K 4096, M 2048: 600 us so, 551 us spread).
-// Measured, us (before: 256 x 128 tiles with the weights staged in LDS as bf16,
-// 128 x 128 below 256 rows, one launch per matrix there):
-//   8-bit, 2 x 14336 x 4096: M 100  88.0 -> 47.2, M 2048  619 -> 520 (925 TFLOP/s)
-//   8-bit, 4096 x 14336:     M 100  44.6 -> 34.3, M 2048  284 -> 235
-//   4-bit, 12352 x 2048:     M 512  41.3 -> 36.2;  9216 x 2048: 39.0 -> 30.5
-//   4-bit, 2048 x 4096:      M 512  26.7 -> 25.4 (with the reduction)
+//     waves at the CU's one address path before their first MFMA (measured while
+//     it was written, 28672 x 4096, 8-bit, M 2048: 600 us so, 551 us spread).
+// Measured, us, a product repeated on the same operands (before: 256 x 128 tiles
+// with the weights staged in LDS as bf16, 128 x 128 below 256 rows):
+//   8-bit, 28672 x 4096: M 100  67.7 -> 44.8, M 2048  537 -> 491 (980 TFLOP/s)
+//   8-bit, 4096 x 14336: M 100  40.9 -> 32.8, M 2048  257 -> 229
+//   4-bit, 12352 x 2048: M 512  37.2 -> 35.4;  2048 x 4096: 32.4 -> 26.8
+// Its fixed cost (fill, sum exchange) is higher: products of several rounds of
+// 256-row tiles with K below about 1300 are slower than they were, 14336 x 640,
+// 8-bit, M 2048: 66.1 -> 72.5; 14336 x 1152, 4-bit, M 2193: 103.2 -> 108.7. One
+// exchange of all the sums instead of four rounds, or three buffers for them,
+// did not shorten it (75.0, 72.6).
 // Within a step, wave k-group kg and lane half h own the run of 16 codes at
 // k = 16 (2 kg + h), and MFMA slice j takes 8 of them: any order of k serves
 // as long as both operands use it.
 // LDS: x rows are 128 bytes, 16-byte granule q of row r at q ^ ((r >> 1) & 7)
-// (16 rows of an operand read spread over all banks: no conflicts counted);
-// 8-bit codes likewise at q ^ ((r >> 2) & 3) of their 64 bytes; the narrower
-// rows need no swizzle.
+// (16 rows of an operand read spread over all banks); 8-bit codes likewise at
+// q ^ ((r >> 2) & 3) of their 64 bytes; the narrower rows are not swizzled.
+// Conflict cycles counted per LDS instruction: none with 128-row 8-bit tiles, 0.6
+// with 256 rows (5 % of the time), 0.3-0.5 at 4 bits.
 constexpr int kTN = 128;   // tile columns
 constexpr int kQMultiMax = 8;
 
@@ -891,13 +899,14 @@ static int qmm_tile_form(const DevMat *ms, int n, int x_stride) {
   return form;
 }
 
-// Tile rows and K split of a product: the least estimated time in us. The
-// constants are fitted to 1,450 measured (M, N, K, bits, rows, split) between
-// 24 and 2048 rows, 1024 and 28672 columns (mean error 6 %; the choice costs
-// 0.2 % over the best one measured): a 64-k step of a block, whose weights
-// are formed whatever its rows, or the time its codes take to arrive; a
-// block's pipeline fill and sum exchange; and for a split its partial sums
-// written and read back and one more launch. One block per CU.
+// Tile rows and K split of a product: the least estimated time in us: a 64-k
+// step of a block, whose weights are formed whatever its rows, or the time its
+// codes take to arrive; a block's pipeline fill and sum exchange; and for a split
+// its partial sums written and read back and one more launch; one block per CU
+// (32-row tiles at 4 and 5 bits would fit two). The fitted constants rank the
+// choices rather than predict the time: over 3,382 measured choices of 273 shapes
+// (24 to 2200 rows, 1000 to 28672 columns) the estimate is 13 % off on average
+// and 11 % low, and the choice costs 0.8 % over the best one measured.
 struct QmmPlan {
   int bm, split;
 };
