@@ -1182,11 +1182,11 @@ __global__ __launch_bounds__(256) void moe_down_mfma_kernel(MoeArgs a, MoeMWs w,
 //     K a multiple of 128 code bytes): 8 waves, each wave a run of 32-row
 //     pairs of 16-row groups. h (hi, lo) is staged once per block (the
 //     register form stages it per 128 rows), and each wave streams its rows'
-//     codes batch by batch through a three-slot ring of RingSlot batches
+//     codes batch by batch through a ring of NB slots of RingSlot batches
 //     (group 0 = rows 32 p + [0, 16), group 1 = rows 32 p + [16, 32) of pair
-//     p), two batches in flight while one is multiplied, the ring running on
+//     p), NB - 1 batches in flight while one is multiplied, the ring running on
 //     from one pair into the next. The sums of h over each step (the fold's
-//     bias term) are formed once and kept.
+//     bias term) are formed once and kept. MT = 1: 16 slots of h, NB = 3.
 //
 //     One block per CU (the ring and the h tile fill its LDS), so blocks run
 //     in rounds and a block's start (h copy, first batches) and end (last
@@ -1200,11 +1200,15 @@ __global__ __launch_bounds__(256) void moe_down_mfma_kernel(MoeArgs a, MoeMWs w,
 //     chunk: 118-119 us per layer with 512-row blocks only, 98 us so; 110 us
 //     with 128 small units, 103 with 512).
 //
-//     MT = 2 (wide tiles, in parts of 32 slots; a two-slot ring): h of 32 rows,
-//     the codes unpacked once for both 16-slot halves. A pair's stores count
-//     in vmcnt behind the copies; waiting for the copies alone made each pair
-//     wait for its own stores too (512-token block 263 -> 258 us, 160 tokens
-//     250 -> 239).
+//     MT = 2 (wide tiles, in parts of 32 slots; NB = 2): h of 32 rows, the
+//     codes unpacked once for both 16-slot halves (a block of 1999 tokens, 512
+//     experts top 10, with the wide tiles in parts of 16 slots -> so: 4-bit
+//     546 -> 487 us, popularity rank^-1.1 643 -> 553, 8-bit 672 -> 629; 683 ->
+//     710 at 8-bit rank^-1.1).
+//     A pair's stores count in vmcnt behind the copies; waiting for the copies
+//     alone made each pair wait for its own stores too (blocks of 160, 512 and
+//     1000 tokens, 4-bit: 231.7 -> 228.6, 258.1 -> 256.0, 383.8 -> 379.4 us;
+//     8-bit 512: 401.4 -> 399.8).
 
 constexpr int kMDownLdsRows = 512;      // rows of a small block (32 x 2 pairs x 8 waves)
 constexpr int kMDownSmallUnits = 256;   // 512-row units left to small blocks (one round on 256 CUs)
@@ -1278,7 +1282,7 @@ __global__ __launch_bounds__(512, 1) void moe_down_lds_kernel(MoeArgs a, MoeMWs 
   // the next batch to copy (uniform): index, ring slot, pair, k batch. Past the
   // wave's last batch the cursor stays there and the copy repeats that batch
   // into its own slot (the same bytes), which keeps the count of copies behind
-  // every batch at 2 NI.
+  // every batch at (NB - 1) NI.
   const uint32_t ring0 = __builtin_amdgcn_readfirstlane(lds_addr(&swt[0][wave][0]));
   int ib = 0, is = 0, ip = 0, ik = 0;
   // the copy sources of pair ip at byte 0 of its rows, formed when the cursor
@@ -1325,7 +1329,7 @@ __global__ __launch_bounds__(512, 1) void moe_down_lds_kernel(MoeArgs a, MoeMWs 
     for (int i = 0; i < NQ; ++i)
       if (NT * i + 64 * wave < cnt * gpr) dma(NT * i + 64 * wave);
   }
-  // the ring's first two batches behind the h copies (a wave with no rows
+  // the ring's first NB - 1 batches behind the h copies (a wave with no rows
   // inside D copies clamped rows and stores nothing)
 #pragma unroll
   for (int i = 0; i < NB - 1; ++i) issue_next();
@@ -1364,10 +1368,9 @@ __global__ __launch_bounds__(512, 1) void moe_down_lds_kernel(MoeArgs a, MoeMWs 
 #pragma unroll
     for (int kb = 0; kb < KBM; ++kb) {
       if (kb < kbn) {
-        // two batches in flight behind this one
-        issue_next();
-        // behind this batch: the copies of the next ones and, in the NB - 1
+        // behind this batch: the copies of the next NB - 1 and, in the NB - 1
         // batches after a pair's stores, those stores
+        issue_next();
         if (p > 0 && kb < NB - 1) lds_dma_wait_behind<(NB - 1) * R::NI + kStores>();
         else lds_dma_wait_behind<(NB - 1) * R::NI>();
         const uint8_t *slot = &swt[cs][wave][0];
@@ -1542,7 +1545,9 @@ static int tiles_bound(const MoeArgs &a, int ts) {
 //  * 32 slots an expert, that is more than two 16-slot tiles (whole block in us,
 //    16-slot -> wide tiles, 512 experts top 10, popularity rank^-1.1: 4-bit 27
 //    an expert 458 -> 472, 39: 587 -> 548; uniform 457 -> 393, 605 -> 482;
-//    8-bit 27: 634 -> 610, 39: 803 -> 703; uniform 666 -> 522, 877 -> 633);
+//    8-bit 27: 634 -> 610, 39: 803 -> 703; uniform 666 -> 522, 877 -> 633: below
+//    the line, which knows the mean alone, only skewed 4-bit routes lose; 8-bit
+//    codes could take a lower one);
 //  * enough (slot, 128-row group) pairs for the 256 CUs, a wide block being
 //    several times as long: 96 each, 60 with 8-bit codes, where the 16-slot
 //    form moves twice the bytes (512 rows: 64 experts top 6, 4-bit 3000 slots
