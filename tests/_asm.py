@@ -1,0 +1,39 @@
+"""The gfx950 assembly of a source and the compiler's resource report, from one
+compilation per source and session."""
+import atexit
+import functools
+import re
+import shutil
+import subprocess
+import tempfile
+from pathlib import Path
+
+from logan_amd import build
+
+CSRC = Path(build.CSRC)
+
+
+@functools.lru_cache(maxsize=None)
+def _dir() -> Path:
+    d = Path(tempfile.mkdtemp(prefix="logan_asm_"))
+    atexit.register(shutil.rmtree, d, ignore_errors=True)
+    return d
+
+
+@functools.lru_cache(maxsize=None)
+def compiled(name: str):
+    """(path of the assembly, {mangled kernel: bytes of scratch per lane})."""
+    out = _dir() / (name + ".s")
+    cmd = [build.hipcc(), *build.HIPFLAGS, "-I", str(build.INCLUDE), "--cuda-device-only", "-S", str(CSRC / name),
+           "-o", str(out), "-Rpass-analysis=kernel-resource-usage"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-2000:]
+    scratch, kernel = {}, None
+    for line in r.stderr.splitlines():
+        m = re.search(r"Function Name: (\S+)", line)
+        if m:
+            kernel = m.group(1)
+        m = re.search(r"ScratchSize \[bytes/lane\]: (\d+)", line)
+        if m and kernel:
+            scratch[kernel] = int(m.group(1))
+    return out, scratch

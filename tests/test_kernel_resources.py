@@ -9,14 +9,13 @@ vector-memory instructions (the tile product, the LDS rings), a spill would
 also break the count.
 """
 import re
-import subprocess
-from pathlib import Path
 
 import pytest
 
 from logan_amd import build
 
-CSRC = Path(build.CSRC)
+from _asm import compiled
+
 HOT = {
     "gemm.hip": [r"affine_qmm_tile_kernelILi%dELi%dE" % (b, mi) for b in (4, 5, 6, 8) for mi in (1, 2, 4, 6, 8)],
     "moe.hip": [r"moe_gateup_kernelILi4ELi1E", r"moe_down_kernelILi4ELi16E", r"moe_route_tok_kernel",
@@ -28,23 +27,6 @@ HOT = {
 }
 
 
-def _scratch_report(src: Path):
-    cmd = [build.hipcc(), *build.HIPFLAGS, "-I", str(build.INCLUDE), "--cuda-device-only", "-c",
-           str(src), "-o", "/dev/null", "-Rpass-analysis=kernel-resource-usage"]
-    r = subprocess.run(cmd, capture_output=True, text=True)
-    assert r.returncode == 0, r.stderr[-2000:]
-    out = {}
-    name = None
-    for line in r.stderr.splitlines():
-        m = re.search(r"Function Name: (\S+)", line)
-        if m:
-            name = m.group(1)
-        m = re.search(r"ScratchSize \[bytes/lane\]: (\d+)", line)
-        if m and name:
-            out[name] = int(m.group(1))
-    return out
-
-
 def test_hot_moe_kernels_use_no_scratch():
     try:
         build.hipcc()
@@ -53,7 +35,7 @@ def test_hot_moe_kernels_use_no_scratch():
     from concurrent.futures import ThreadPoolExecutor
 
     with ThreadPoolExecutor(len(HOT)) as ex:
-        reps = dict(zip(sorted(HOT), ex.map(lambda s: _scratch_report(CSRC / s), sorted(HOT))))
+        reps = dict(zip(sorted(HOT), ex.map(lambda s: compiled(s)[1], sorted(HOT))))
     for src, pats in HOT.items():
         for pat in pats:
             hits = {k: v for k, v in reps[src].items() if re.search(pat, k)}

@@ -13,23 +13,17 @@ that a wave may still have in flight (they return in order; lgkmcnt(n) leaves
 the last n).
 """
 import re
-import subprocess
-from pathlib import Path
 
 import pytest
 
 from logan_amd import build
 
-CSRC = Path(build.CSRC)
+from _asm import compiled
 
 
-def _kernels(src: Path, pattern: str, tmp: Path):
+def _kernels(name: str, pattern: str):
     """{mangled name: instruction and label lines} of the kernels matching."""
-    out = tmp / (src.stem + ".s")
-    cmd = [build.hipcc(), *build.HIPFLAGS, "-I", str(build.INCLUDE), "--cuda-device-only", "-S", str(src),
-           "-o", str(out)]
-    r = subprocess.run(cmd, capture_output=True, text=True)
-    assert r.returncode == 0, r.stderr[-2000:]
+    out = compiled(name)[0]
     found, cur = {}, None
     with open(out) as f:
         for line in f:
@@ -119,11 +113,11 @@ def test_the_walk_itself():
     assert reads_in_flight(code, "s_barrier") == (0, 2)
 
 
-def test_qmm_tile_reads_complete_at_the_barriers(hipcc, tmp_path):
+def test_qmm_tile_reads_complete_at_the_barriers(hipcc):
     """Of the tile product's LDS reads only the last ones, the MI reads of the
     next slice's x operands, may be in flight at a barrier: the copies behind
     it overwrite the codes just read, and x of a step before those."""
-    ks = _kernels(CSRC / "gemm.hip", "affine_qmm_tile_kernel", tmp_path)
+    ks = _kernels("gemm.hip", "affine_qmm_tile_kernel")
     assert ks
     bad = {}
     for name, lines in ks.items():
@@ -135,10 +129,10 @@ def test_qmm_tile_reads_complete_at_the_barriers(hipcc, tmp_path):
     assert not bad
 
 
-def test_moe_ring_reads_complete_at_the_copies(hipcc, tmp_path):
+def test_moe_ring_reads_complete_at_the_copies(hipcc):
     """A wave's reads of its ring complete before it copies the next batch
     into the slot it has read."""
-    ks = _kernels(CSRC / "moe_mfma.hip", "(lds|wide)_kernel", tmp_path)
+    ks = _kernels("moe_mfma.hip", "(lds|wide)_kernel")
     assert ks
     bad = {}
     for name, lines in ks.items():
