@@ -230,7 +230,8 @@ static SlotRing g_qmm_slots(kQSlots);
 
 // ---------------------------------------------------------------------------
 // Products of up to kQMultiMax matrices that read the same x (q/k/v, qkvz/ba,
-// gate/up) in one grid, BM x 128 output tiles, one 8-wave block per CU.
+// gate/up) in one grid, BM x 128 output tiles, one 8-wave block per CU (two of
+// 32-row tiles).
 //
 // What bounds it: 256-row tiles the matrix and vector pipes, which hardly
 // overlap (8-bit, 2 x 14336 columns, K 4096, M 2048: of 2,090 cycles per 64-k
@@ -330,15 +331,23 @@ struct QTile {
   static constexpr int RB = 8 * BITS;              // code bytes per row and step
   static constexpr int XB = BM * 128;              // x bytes per stage
   static constexpr int WB = kTN * RB;
-  // stages of x and of the codes (a step's codes are read a step ahead of its x)
-  static constexpr int NST = BM >= 192 ? 4 : BM == 128 ? 5 : 8;
-  static constexpr int NWS = NST - 1;
-  static constexpr int AUX0 = NST * XB + NWS * WB;
+  // LDS of a block: 32-row tiles leave room for a second one on the CU. With one,
+  // products of few rows and more than 256 column tiles ran in full rounds (8 and
+  // 6 bits with 8 stages, M 5, us, 64 x 64 kernel / so / with a second block:
+  // 33000 x 1024 15 / 19 / 14, 100000 x 2304 68 / 75 / 54, 152064 x 4096 266 /
+  // 166 / 154; 256 tiles or fewer the same: 28672 x 4096 47 / 31 / 31).
+  static constexpr int LIM = BM == 32 ? 81920 : 163840;
   // steps of a chunk of scale / bias words, dwords per row of it: CS groups of
   // 64 that may start inside a dword; groups of 32 start on one (when ALN)
   static constexpr int ndw(int cs) { return GS64 ? cs / 2 + 1 : cs + !ALN; }
   static constexpr int ab(int cs) { return 2 * kTN * ndw(cs) * 4; }  // [scale, bias][128][ndw]
-  static constexpr int CS = AUX0 + 2 * ab(8) <= 163840 ? 8 : AUX0 + 2 * ab(6) <= 163840 ? 6 : 4;
+  // stages of x and of the codes (a step's codes are read a step ahead of its x)
+  static constexpr int rings(int nst) { return nst * XB + (nst - 1) * WB; }
+  static constexpr int fit(int nst) { return rings(nst) + 2 * ab(8) <= LIM ? nst : fit(nst - 1); }
+  static constexpr int NST = BM >= 192 ? 4 : BM == 128 ? 5 : BM == 64 ? 8 : fit(8);
+  static constexpr int NWS = NST - 1;
+  static constexpr int AUX0 = rings(NST);
+  static constexpr int CS = AUX0 + 2 * ab(8) <= LIM ? 8 : AUX0 + 2 * ab(6) <= LIM ? 6 : 4;
   static constexpr int NDW = ndw(CS);
   static constexpr int AB = ab(CS);
   static constexpr int XI = BM / 8;                // x copies (1 KB) of a stage
@@ -352,7 +361,7 @@ struct QTile {
   // sum exchange: a 32 x 32 tile per wave; stores: one of 33-float rows
   static constexpr int ROUND = 8 * 4096 + 8 * 32 * 33 * 4;
   static constexpr int BYTES = RINGS > ROUND ? RINGS : ROUND;
-  static_assert(BYTES <= 163840 && CS >= NST, "ring geometry");
+  static_assert(BYTES <= LIM && CS >= NST, "ring geometry");
   static_assert((NST - 2) * L + NA <= 63, "vmcnt is 6 bits");
 };
 
@@ -903,7 +912,8 @@ static int qmm_tile_form(const DevMat *ms, int n, int x_stride) {
 // step of a block, whose weights are formed whatever its rows, or the time its
 // codes take to arrive; a block's pipeline fill and sum exchange; and for a split
 // its partial sums written and read back and one more launch; one block per CU
-// (32-row tiles at 4 and 5 bits would fit two). The fitted constants rank the
+// (of 32-row tiles it holds two, which take about half again as long as one:
+// nearer to one round than to the two counted). The fitted constants rank the
 // choices rather than predict the time: over 3,382 measured choices of 273 shapes
 // (24 to 2200 rows, 1000 to 28672 columns) the estimate is 13 % off on average
 // and 11 % low, and the choice costs 0.8 % over the best one measured.

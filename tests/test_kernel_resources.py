@@ -40,5 +40,18 @@ def test_hot_moe_kernels_use_no_scratch():
         for pat in pats:
             hits = {k: v for k, v in reps[src].items() if re.search(pat, k)}
             assert hits, f"no kernel matches {pat} in {src}"
-            bad = {k: v for k, v in hits.items() if v != 0}
+            bad = {k: v for k, v in hits.items() if v["ScratchSize [bytes/lane]"] != 0}
             assert not bad, f"scratch in {src}: {bad}"
+
+
+def test_tile_product_of_32_rows_fits_two_blocks_a_cu():
+    """Products of few rows and 257 to 512 column tiles run in one round only
+    if a CU holds two blocks: half of its LDS, and 128 registers a thread."""
+    try:
+        build.hipcc()
+    except RuntimeError:
+        pytest.skip("hipcc not available")
+    ks = {k: v for k, v in compiled("gemm.hip")[1].items() if re.search(r"affine_qmm_tile_kernelILi\dELi1E", k)}
+    assert len(ks) == 24
+    bad = {k: v for k, v in ks.items() if v["LDS Size [bytes/block]"] > 81920 or v["VGPRs"] > 128}
+    assert not bad
