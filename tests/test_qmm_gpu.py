@@ -524,3 +524,49 @@ def test_qmm_tile_forms(gpu, rows, M, bits):
         assert qmm_route([part], 64)[0] == 0
         y64 = affine_qmm(part, x[:64], out_dtype=torch.float32)
         assert float((y64 - y[:64, :n]).abs().max() / y64.abs().max()) <= 1e-5
+
+
+def test_tile_products_in_a_graph(gpu):
+    """Tile products (one k range and several, one matrix and several, the
+    dword form) captured in one graph: every replay, with eager products and
+    synchronisations between, gives the eager bits."""
+    import torch
+    from logan_amd.device import AffineMatrix, affine_qmm, affine_qmm_multi
+
+    jobs = []
+    for M, Os, I, bits, off in [(512, (512,), 2048, 4, 0), (270, (200, 130), 2048, 6, 0), (100, (4096,), 1024, 8, 2),
+                                (300, (12352,), 512, 4, 0), (200, (1000,), 2880, 8, 2)]:
+        rng = np.random.default_rng(M + I)
+        mats = [dev_matrix(torch, *make_affine(rng, O, I, bits, 64), O, I, bits, 64) for O in Os]
+        if off:
+            mats = [AffineMatrix(m.weights, shifted(torch, m.scales, off), shifted(torch, m.biases, off), m.O, I, bits,
+                                 64, False) for m in mats]
+        x = to_dev(make_x(rng, M, I).reshape(M, I).view(np.int16), torch).view(torch.bfloat16)
+        assert qmm_route(mats, M)[0] == (2 if off else 1)
+        jobs.append((mats, x, [torch.empty((M, O), device="cuda") for O in Os]))
+    splits = [qmm_route(mats, x.shape[0])[2] for mats, x, _ in jobs]
+    assert min(splits) == 1 and max(splits) > 1
+
+    def step():
+        for mats, x, ys in jobs:
+            if len(mats) > 1:
+                affine_qmm_multi(mats, x, outs=ys)
+            else:
+                affine_qmm(mats[0], x, out=ys[0])
+
+    step()
+    torch.cuda.synchronize()
+    want = [[y.clone() for y in ys] for _, _, ys in jobs]
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        step()
+    for _ in range(4):
+        for _, _, ys in jobs:
+            for y in ys:
+                y.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        for (_, _, ys), ws in zip(jobs, want):
+            assert all(torch.equal(y, w) for y, w in zip(ys, ws))
+        step()
+        torch.cuda.synchronize()
