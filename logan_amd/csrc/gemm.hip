@@ -255,14 +255,9 @@ static SlotRing g_qmm_slots(kQSlots);
 //     it was written, 28672 x 4096, 8-bit, M 2048: 600 us so, 551 us spread).
 // Measured, us, a product repeated on the same operands (before: 256 x 128 tiles
 // with the weights staged in LDS as bf16, 128 x 128 below 256 rows):
-//   8-bit, 28672 x 4096: M 100  67.7 -> 44.8, M 2048  537 -> 491 (980 TFLOP/s)
-//   8-bit, 4096 x 14336: M 100  40.9 -> 32.8, M 2048  257 -> 229
-//   4-bit, 12352 x 2048: M 512  37.2 -> 35.4;  2048 x 4096: 32.4 -> 26.8
-// Its fixed cost (fill, sum exchange) is higher: products of several rounds of
-// 256-row tiles with K below about 1300 are slower than they were, 14336 x 640,
-// 8-bit, M 2048: 66.1 -> 72.5; 14336 x 1152, 4-bit, M 2193: 103.2 -> 108.7. One
-// exchange of all the sums instead of four rounds, or three buffers for them,
-// did not shorten it (75.0, 72.6).
+//   8-bit, 28672 x 4096: M 100  66.0 -> 39.3, M 2048  522 -> 467 (1030 TFLOP/s)
+//   8-bit, 4096 x 14336: M 100  40.0 -> 31.6, M 2048  251 -> 220
+//   4-bit, 12352 x 2048: M 512  36.8 -> 32.9;  2048 x 4096: 30.1 -> 26.2
 // Within a step, wave k-group kg and lane half h own the run of 16 codes at
 // k = 16 (2 kg + h), and MFMA slice j takes 8 of them: any order of k serves
 // as long as both operands use it.
@@ -727,49 +722,76 @@ __global__ __launch_bounds__(512, 2) void affine_qmm_tile_kernel(QmmMulti p, int
 
   // ---- sums of the two waves of a tile, added in k order, and stores ----
   // Element e of a 32 x 32 tile in lane l: column (m) l % 32, row (n)
-  // 8 (e / 4) + 4 (l / 32) + e % 4, so a lane stores 4 consecutive columns of
-  // y at a time. Row tile i is summed and stored by k-group i % 2.
+  // 8 (e / 4) + 4 (l / 32) + e % 4. A wave turns its tile through LDS, so that a
+  // store instruction writes whole runs of 64 (bf16) or 128 bytes of y's rows;
+  // straight from the sums it writes 16 or 32 bytes in each of 32 rows. Nothing
+  // overlaps a block's stores (16384 columns, M 2048, 8-bit, us, without sums and
+  // stores / straight / turned: K 512 38.8 / 64.1 / 56.6, K 2048 131.8 / 155.0 /
+  // 147.9; f32 partial sums the same either way).
+  // Row tile i is summed and stored by k-group i % 2.
   const bool split = slot >= 0;
   float *part = split ? g_qmm_part + (size_t)slot * kQSlotFloats + (size_t)z * p.M * p.part_N + mat.col0
                       : nullptr;
   float *const flat = reinterpret_cast<float *>(smem + 32768 + wave * (32 * 33 * 4));
+  auto turned = [&]() __attribute__((always_inline)) {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_wave_barrier();
+  };
   auto store = [&](int i, const f32x16 &v) {
-    const int m = bm0 + 32 * i + l32, nw = bn0 + wn * 32;
-    if (split || p.vec) {
-      if (m >= p.M) return;
+    const int nw = bn0 + wn * 32;
+    if (split || (p.vec && !p.y_bf16)) {
+      // 16-byte granule c of row r at c ^ (r & 7) of its 128 bytes
+      float4 *const t = reinterpret_cast<float4 *>(flat);
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        t[8 * l32 + ((2 * q + half) ^ (l32 & 7))] = make_float4(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]);
+      turned();
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const int n = nw + 8 * q + 4 * half;
-        const float fe[4] = {v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
-        if (split || !p.y_bf16) {
-          float *dst = split ? part + (size_t)m * p.part_N + n
-                             : reinterpret_cast<float *>(mat.y) + (size_t)m * mat.y_stride + n;
-          if (n + 4 <= (split ? (N + 3) & ~3 : N)) {
-            *reinterpret_cast<float4 *>(dst) = make_float4(fe[0], fe[1], fe[2], fe[3]);
-          } else {
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-              if (n + e < N) dst[e] = fe[e];
-          }
+        const int r = 8 * q + (lane >> 3), c = lane & 7;
+        const int m = bm0 + 32 * i + r, n = nw + 4 * c;
+        const float4 f = t[8 * r + (c ^ (r & 7))];
+        if (m >= p.M) continue;
+        float *dst = split ? part + (size_t)m * p.part_N + n
+                           : reinterpret_cast<float *>(mat.y) + (size_t)m * mat.y_stride + n;
+        if (n + 4 <= (split ? (N + 3) & ~3 : N)) {
+          *reinterpret_cast<float4 *>(dst) = f;
         } else {
-          __bf16 *dst = reinterpret_cast<__bf16 *>(mat.y) + (size_t)m * mat.y_stride + n;
-          if (n + 4 <= N) {
-            typedef __bf16 b4 __attribute__((ext_vector_type(4)));
-            *reinterpret_cast<b4 *>(dst) = b4{(__bf16)fe[0], (__bf16)fe[1], (__bf16)fe[2], (__bf16)fe[3]};
-          } else {
+          const float fe[4] = {f.x, f.y, f.z, f.w};
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
-              if (n + e < N) dst[e] = (__bf16)fe[e];
-          }
+          for (int e = 0; e < 4; ++e)
+            if (n + e < N) dst[e] = fe[e];
+        }
+      }
+    } else if (p.vec) {
+      // 16-byte granule c of row r at c ^ ((r >> 2) & 3) of its 64 bytes
+      typedef __bf16 b4 __attribute__((ext_vector_type(4)));
+      typedef __bf16 b8 __attribute__((ext_vector_type(8)));
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        reinterpret_cast<b4 *>(flat)[8 * l32 + 2 * (q ^ ((l32 >> 2) & 3)) + half] =
+            b4{(__bf16)v[4 * q], (__bf16)v[4 * q + 1], (__bf16)v[4 * q + 2], (__bf16)v[4 * q + 3]};
+      turned();
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const int r = 16 * q + (lane >> 2), c = lane & 3;
+        const int m = bm0 + 32 * i + r, n = nw + 8 * c;
+        const b8 f = reinterpret_cast<const b8 *>(flat)[4 * r + (c ^ ((r >> 2) & 3))];
+        if (m >= p.M) continue;
+        __bf16 *dst = reinterpret_cast<__bf16 *>(mat.y) + (size_t)m * mat.y_stride + n;
+        if (n + 8 <= N) {
+          *reinterpret_cast<b8 *>(dst) = f;
+        } else {
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+            if (n + e < N) dst[e] = f[e];
         }
       }
     } else {
-      // rows off 16 bytes: element stores of 32 consecutive columns, the tile
-      // turned through LDS
+      // rows off 16 bytes: element stores of 32 consecutive columns
 #pragma unroll
       for (int e = 0; e < 16; ++e) flat[l32 * 33 + 8 * (e / 4) + 4 * half + e % 4] = v[e];
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      __builtin_amdgcn_wave_barrier();
+      turned();
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
         const int row = 2 * e + half, mm = bm0 + 32 * i + row, n = nw + l32;

@@ -55,3 +55,28 @@ def test_tile_product_of_32_rows_fits_two_blocks_a_cu():
     assert len(ks) == 24
     bad = {k: v for k, v in ks.items() if v["LDS Size [bytes/block]"] > 81920 or v["VGPRs"] > 128}
     assert not bad
+
+
+def test_tile_product_stores_whole_runs():
+    """Aligned rows of y are stored 16 bytes a lane, the tile turned through
+    LDS; 8-byte stores are those of the sums' own layout (bf16), 16 bytes in
+    each of 32 rows per instruction."""
+    try:
+        build.hipcc()
+    except RuntimeError:
+        pytest.skip("hipcc not available")
+    stores, kernel = {}, None
+    with open(compiled("gemm.hip")[0]) as f:
+        for line in f:
+            m = re.match(r"(_ZN\S*affine_qmm_tile_kernel\S+):", line)
+            if m:
+                kernel = stores.setdefault(m[1], [])
+            elif line.startswith(".Lfunc_end"):
+                kernel = None
+            elif kernel is not None:
+                m = re.match(r"\s+(global_store\w+)", line)
+                if m:
+                    kernel.append(m[1])
+    assert len(stores) == 119
+    for name, ops in stores.items():
+        assert "global_store_dwordx4" in ops and "global_store_dwordx2" not in ops, name
