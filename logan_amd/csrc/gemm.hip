@@ -234,11 +234,11 @@ static SlotRing g_qmm_slots(kQSlots);
 // 32-row tiles).
 //
 // What bounds it: 256-row tiles the matrix and vector pipes, which hardly
-// overlap (8-bit, 2 x 14336 columns, K 4096, M 2048: of 2,090 cycles per 64-k
+// overlap (8-bit, 2 x 14336 columns, K 4096, M 2048: of 2,040 cycles per 64-k
 // step a SIMD's matrix pipe is busy 1,024 and its vector pipe 690, most of it
-// the forming of the bf16 weights, at the 1.8-1.86 GHz the card holds under this
+// the forming of the bf16 weights, at the 1.8-1.9 GHz the card holds under this
 // load); tiles of at most 128 rows a step's chain of LDS reads, forming, MFMAs
-// and barrier with two waves a SIMD (M 100: 1,830 cycles for 512 and 510), the
+// and barrier with two waves a SIMD (M 100: 1,760 cycles for 512 and 590), the
 // codes arriving at 2.7 TB/s. Hence:
 //   * every copy from memory goes straight into LDS (global_load_lds, issued
 //     through inline assembly and waited for by count) NST - 1 steps ahead: x
@@ -264,8 +264,8 @@ static SlotRing g_qmm_slots(kQSlots);
 // LDS: x rows are 128 bytes, 16-byte granule q of row r at q ^ ((r >> 1) & 7)
 // (16 rows of an operand read spread over all banks); 8-bit codes likewise at
 // q ^ ((r >> 2) & 3) of their 64 bytes; the narrower rows are not swizzled.
-// Conflict cycles counted per LDS instruction: none with 128-row 8-bit tiles, 0.6
-// with 256 rows (5 % of the time), 0.3-0.5 at 4 bits.
+// Conflict cycles counted per LDS instruction: none with 128-row 8-bit tiles, 0.66
+// with 256 rows (5 % of the time), 0.4-0.5 at 4 bits.
 constexpr int kTN = 128;   // tile columns
 constexpr int kQMultiMax = 8;
 
@@ -937,8 +937,8 @@ static int qmm_tile_form(const DevMat *ms, int n, int x_stride) {
 // (of 32-row tiles it holds two, which take about half again as long as one:
 // nearer to one round than to the two counted). The fitted constants rank the
 // choices rather than predict the time: over 3,382 measured choices of 273 shapes
-// (24 to 2200 rows, 1000 to 28672 columns) the estimate is 13 % off on average
-// and 11 % low, and the choice costs 0.8 % over the best one measured.
+// (24 to 2200 rows, 1000 to 28672 columns) the estimate is 11 % off on average
+// and 7 % low, and the choice costs 0.3 % over the best one measured, 12 % at most.
 struct QmmPlan {
   int bm, split;
 };
