@@ -983,8 +983,8 @@ static QmmRoute qmm_route(const DevMat *ms, int n, int x_stride, int M) {
                      (long long)ms[0].O * ms[0].I <= (10 << 20);
   // By dwords above 64 rows only: up to there the 64 x 64 kernel forms every
   // weight once as well. 4096 x 4096, 8-bit, 64 x 64 kernel / tile kernel by
-  // dwords, us: sidecars off 4 bytes, M 100: 29.5 / 20.7, 512: 81.9 / 37.3,
-  // 2048: 286 / 74; 4-bit weights off 16 bytes: 30.2 / 22.1, 79.8 / 36.0, 281 / 74.
+  // dwords, us: sidecars off 4 bytes, M 100: 29.5 / 20.8, 512: 81.9 / 38.7,
+  // 2048: 286 / 74; 4-bit weights off 16 bytes: 30.2 / 22.5, 79.8 / 36.6, 281 / 73.
   const int form = small ? kQNone : qmm_tile_form(ms, n, x_stride);
   if (form == kQNone || (form == kQDword && M <= kTile)) return QmmRoute{kQNone, 0, 0};
   int tiles = 0, cols = 0;
